@@ -19,9 +19,10 @@
 //    are 16-byte channel chunks of neighbouring voxels read from there (1 KB per
 //    instruction, conflict-free), B fragments 16-byte chunks of the weights.  Bias, ReLU
 //    and the ReLU-derivative mask of the data gradient are fused into the epilogue.
-//  * The 1->32 and 32->1 layers and all weight gradients run on the VALU in FP32
-//    (they are 64x smaller or reduction-shaped); weight gradients reduce per block in
-//    registers and once per block with FP32 atomics.
+//  * The 32->32 weight gradients are GEMMs over the voxels on the same instruction,
+//    their operands transposed by the LDS reads.
+//  * The 1->32 and 32->1 layers and their weight gradients run on the VALU in FP32 (they
+//    are 32x smaller).
 #include "common.h"
 
 #include <cfloat>
@@ -262,121 +263,290 @@ __global__ __launch_bounds__(256) void conv_out_bwd_data_kernel(const float * __
 }
 
 // --------------------------------------------------------- weight gradients
-// Grid-stride over voxels; every block accumulates its share in registers and
-// adds it to the FP32 gradient once with atomics.
+// Persistent workgroups: each walks every gridDim.x-th tile of 16 (x) x 4 (y) x 4 (z)
+// voxels with its sums in registers and writes them once, to its own slice of `part`;
+// wgrad_reduce_kernel adds the slices in a fixed order, so the gradients are the same
+// from run to run (per-workgroup atomics on the 27.7k sums of a layer were not).
 
-// dW[t][co][ci] += sum_v dz[v][co] a[v + d(t)][ci];  db[co] += sum_v dz[v][co]
-// thread: co = tid / 8, ci = 4 (tid % 8) .. +3, all 27 taps.
-__global__ __launch_bounds__(256) void wgrad32_kernel(const bf16_t * __restrict__ a, const bf16_t * __restrict__ dz,
-                                                       float * __restrict__ dW, float * __restrict__ db, int B, int X,
-                                                       int Y, int Z)
+// Tile `tile` of the batch: its voxel origin and the base of its volume.
+struct WgTile
 {
-  const int  co = threadIdx.x >> 3, ci0 = 4 * (threadIdx.x & 7);
-  const long n = long(B) * X * Y * Z;
-  float      acc[T][4];
-  float      accb = 0.f;
+  int  x0, y0, z0;
+  long vol;
+};
+__device__ __forceinline__ WgTile
+WgTileOf(int tile, int X, int Y, int Z, int tilesX, int tilesY, int tilesZ)
+{
+  WgTile r;
+  r.x0 = (tile % tilesX) * 16;
+  tile /= tilesX;
+  r.y0 = (tile % tilesY) * 4;
+  tile /= tilesY;
+  r.z0 = (tile % tilesZ) * 4;
+  r.vol = long(tile / tilesZ) * X * Y * Z;
+  return r;
+}
+
+typedef short    short4v __attribute__((ext_vector_type(4)));
+typedef short    short8v __attribute__((ext_vector_type(8)));
+using LdsShort4 = __attribute__((address_space(3))) short4v;
+
+// Four 16-bit channels of four voxels, transposed by the LDS read: in each group of 16
+// lanes, lane i points at 8 bytes, channels 4 (i % 4) .. + 3 of voxel i / 4, and receives
+// channel i of the voxels 0..3 (ds_read_b64_tr_b16).
+__device__ __forceinline__ short4v
+LdsTranspose(const short * p)
+{
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4 *)(p));
+}
+
+// dW[t][co][ci] = sum_v dz[v][co] a[v + d(t)][ci];  db[co] = sum_v dz[v][co].
+// A GEMM per tap with the voxels as the contracted index: M = co, N = ci, K = 32 voxels
+// (two x rows of the tile) per v_mfma_f32_16x16x32_bf16.  Activations are channels-last,
+// so both operands are wanted transposed (eight voxels of one channel per lane); the
+// transposing LDS read delivers them from the tile as it lies in memory, for every tap
+// shift alike (a shift moves the voxel rows, never the alignment).  Both operands take
+// the same voxel order inside K, which is all the product needs.
+// The tile's a with a one-voxel halo (41.5 KB) and its dz (16 KB) are staged in LDS: two
+// workgroups per CU, one loading while the other multiplies.  Wave w takes the taps
+// w, w + 4, ..: 7 x 2 x 2 accumulators of 4 FP32 registers; wave 3, with six taps, also
+// sums dz (a product with ones).  Voxels outside the volume are zeros in both operands.
+// Bound by the LDS reads (a 2 KB operand per 4 matrix instructions) and the staging.
+// 4 x 64^3 voxels, one layer: 11.1 ms (one FMA per voxel, tap and channel pair on the
+// VALU, every operand from global memory) -> 0.11 ms, and 0.04 ms for the slices.
+constexpr int kWgSums = T * C * C + C; // sums of a 32 -> 32 layer
+
+__global__ __launch_bounds__(256) void wgrad32_mfma_kernel(const bf16_t * __restrict__ a,
+                                                            const bf16_t * __restrict__ dz, float * __restrict__ part,
+                                                            int X, int Y, int Z, int tilesX, int tilesY, int tilesZ,
+                                                            int ntiles)
+{
+  constexpr int HX = 18, HY = 6, HZ = 6, NCHUNK = HX * HY * HZ * 4;
+  __shared__ bf16x8 halo[NCHUNK];
+  __shared__ bf16x8 dzt[256 * 4];
+  const short * hs = reinterpret_cast<const short *>(halo);
+  const short * ds = reinterpret_cast<const short *>(dzt);
+  const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // this lane's source address inside an x row of voxels: voxel, first channel
+  const int     src = (4 * (lane >> 4) + ((lane & 15) >> 2)) * C + 4 * (lane & 3);
+  const bf16x8  zero8 = bf16x8{ bf16_t(0.f), bf16_t(0.f), bf16_t(0.f), bf16_t(0.f),
+                               bf16_t(0.f), bf16_t(0.f), bf16_t(0.f), bf16_t(0.f) };
+  const bf16x8  one8 = bf16x8{ bf16_t(1.f), bf16_t(1.f), bf16_t(1.f), bf16_t(1.f),
+                              bf16_t(1.f), bf16_t(1.f), bf16_t(1.f), bf16_t(1.f) };
+  floatx4       acc[7][2][2];
+#pragma unroll
+  for (int i = 0; i < 7; i++)
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      acc[i][m >> 1][m & 1] = floatx4{ 0.f, 0.f, 0.f, 0.f };
+
+  // K = 32 voxels: x rows y and y + 1 of plane z; `row` is the offset of the first
+  auto frag = [&](const short * base, int row, int rowStep, int half) {
+    const short4v lo = LdsTranspose(base + row + src + 16 * half);
+    const short4v hi = LdsTranspose(base + row + rowStep + src + 16 * half);
+    const short8v v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, v);
+  };
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
+  {
+    const WgTile w = WgTileOf(tile, X, Y, Z, tilesX, tilesY, tilesZ);
+    __syncthreads(); // the previous tile's reads are done
+    for (int c = threadIdx.x; c < NCHUNK; c += 256)
+    {
+      const int part8 = c & 3, vi = c >> 2;
+      const int xs = w.x0 - 1 + vi % HX, ys = w.y0 - 1 + (vi / HX) % HY, zs = w.z0 - 1 + vi / (HX * HY);
+      bf16x8    v = zero8;
+      if (xs >= 0 && xs < X && ys >= 0 && ys < Y && zs >= 0 && zs < Z)
+        v = *reinterpret_cast<const bf16x8 *>(a + ((w.vol + (long(zs) * Y + ys) * X + xs) * C + 8 * part8));
+      halo[c] = v;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+    {
+      const int c = threadIdx.x + 256 * q, part8 = c & 3, vi = c >> 2;
+      const int xs = w.x0 + (vi & 15), ys = w.y0 + ((vi >> 4) & 3), zs = w.z0 + (vi >> 6);
+      bf16x8    v = zero8;
+      if (xs < X && ys < Y && zs < Z)
+        v = *reinterpret_cast<const bf16x8 *>(dz + ((w.vol + (long(zs) * Y + ys) * X + xs) * C + 8 * part8));
+      dzt[c] = v;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s < 8; s++)
+    {
+      const int    z = s >> 1, y = 2 * (s & 1);
+      const bf16x8 a0 = frag(ds, (z * 4 + y) * 16 * C, 16 * C, 0), a1 = frag(ds, (z * 4 + y) * 16 * C, 16 * C, 1);
+#pragma unroll
+      for (int i = 0; i < 7; i++)
+      {
+        const int t = wave + 4 * i; // uniform; t = 27 (wave 3 only): the sum of dz
+        bf16x8    b0 = one8, b1 = one8;
+        if (t < T)
+        {
+          const int row = (((z + t / 9) * HY + y + (t / 3) % 3) * HX + t % 3) * C;
+          b0 = frag(hs, row, HX * C, 0);
+          b1 = frag(hs, row, HX * C, 1);
+        }
+        acc[i][0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[i][0][0], 0, 0, 0);
+        acc[i][0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[i][0][1], 0, 0, 0);
+        acc[i][1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[i][1][0], 0, 0, 0);
+        acc[i][1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[i][1][1], 0, 0, 0);
+      }
+    }
+  }
+  // D layout: rows (co) 4 (lane / 16) + q, column (ci) lane % 16
+  float * dst = part + size_t(blockIdx.x) * kWgSums;
+#pragma unroll
+  for (int i = 0; i < 7; i++)
+  {
+    const int t = wave + 4 * i;
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+      {
+        const int   co = 16 * (m >> 1) + 4 * (lane >> 4) + q, ci = 16 * (m & 1) + (lane & 15);
+        const float v = acc[i][m >> 1][m & 1][q];
+        if (t < T)
+          dst[(t * C + co) * C + ci] = v;
+        else if (ci == 0) // every column holds the sum of dz
+          dst[T * C * C + co] = v;
+      }
+  }
+}
+
+// The layers with one channel on one side, as sums over voxels of a 32-channel BF16 field
+// m and an FP32 scalar field f:  S[t][c] = sum_v m[v][c] f[v + d(t)].
+//   layer 1: dW1[t][c] = s S[t][c] with m = dz1, f = x;  db1[c] = sum_v m[v][c]
+//   layer 6: dW6[t][c] = S[26 - t][c] / s with m = a5, f = dy;  db6 = sum_v f[v] / s
+// (v + d(t) = u  <=>  u + d(26 - t) = v).
+// FP32 on the VALU: a thread is one channel, a half-wave the 32 channels of one voxel, 8
+// half-waves the tile's 16 x rows, two each.  f with its halo is staged in LDS and read
+// as broadcast rows of 18 values: 5 LDS reads feed 48 FMAs.  VALU-bound (27 FMAs per
+// voxel and channel).  4 x 64^3 voxels: 1.21 / 1.24 ms (layers 1 / 6; operands from
+// global memory, one voxel a workgroup step) -> 0.09 ms.
+constexpr int kWgIoSums = T * C + C + 1; // S, sum of m per channel, sum of f
+
+__global__ __launch_bounds__(256) void wgrad_io_kernel(const float * __restrict__ f, const bf16_t * __restrict__ m,
+                                                        float * __restrict__ part, int X, int Y, int Z, int tilesX,
+                                                        int tilesY, int tilesZ, int ntiles)
+{
+  constexpr int HX = 20, HY = 6, HZ = 6; // rows padded from 18 to 20 floats: 16-byte reads
+  __shared__ __align__(16) float fh[HX * HY * HZ];
+  __shared__ float               red[8][T + 2][C];
+  const int c = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  float     acc[T], accm = 0.f, accf = 0.f;
 #pragma unroll
   for (int t = 0; t < T; t++)
-    for (int e = 0; e < 4; e++)
-      acc[t][e] = 0.f;
-  for (long v = blockIdx.x; v < n; v += gridDim.x)
+    acc[t] = 0.f;
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
   {
-    const int   i = int(v % X), j = int((v / X) % Y), k = int((v / (long(X) * Y)) % Z);
-    const float g = float(dz[v * C + co]);
-    accb += g;
-#pragma unroll
-    for (int t = 0; t < T; t++)
+    const WgTile w = WgTileOf(tile, X, Y, Z, tilesX, tilesY, tilesZ);
+    __syncthreads();
+    for (int q = threadIdx.x; q < HX * HY * HZ; q += 256)
     {
-      int       dx, dy, dzz;
-      const int off = TapOffset(t, X, Y, dx, dy, dzz);
-      if (i + dx >= 0 && i + dx < X && j + dy >= 0 && j + dy < Y && k + dzz >= 0 && k + dzz < Z)
-      {
-        const bf16_t * s = a + (v + off) * C + ci0;
+      const int xs = w.x0 - 1 + q % HX, ys = w.y0 - 1 + (q / HX) % HY, zs = w.z0 - 1 + q / (HX * HY);
+      fh[q] = (q % HX < 18 && xs >= 0 && xs < X && ys >= 0 && ys < Y && zs >= 0 && zs < Z)
+                ? f[w.vol + (long(zs) * Y + ys) * X + xs]
+                : 0.f;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int r = grp; r < 16; r += 8)
+    {
+      const int y = r & 3, z = r >> 2;
+      if (w.y0 + y >= Y || w.z0 + z >= Z)
+        continue;
+      const bf16_t * src = m + (w.vol + (long(w.z0 + z) * Y + w.y0 + y) * X + w.x0) * C + c;
+      float          mv[16];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          acc[t][e] += g * float(s[e]);
+      for (int x = 0; x < 16; x++)
+        mv[x] = w.x0 + x < X ? float(src[x * C]) : 0.f;
+#pragma unroll
+      for (int x = 0; x < 16; x++)
+        accm += mv[x];
+#pragma unroll
+      for (int l = 0; l < 9; l++)
+      {
+        const float4 * row = reinterpret_cast<const float4 *>(fh + ((z + l / 3) * HY + y + l % 3) * HX);
+        float          fv[20];
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+        {
+          const float4 v = row[q];
+          fv[4 * q] = v.x;
+          fv[4 * q + 1] = v.y;
+          fv[4 * q + 2] = v.z;
+          fv[4 * q + 3] = v.w;
+        }
+#pragma unroll
+        for (int x = 0; x < 16; x++)
+#pragma unroll
+          for (int d = 0; d < 3; d++)
+            acc[3 * l + d] = fmaf(mv[x], fv[x + d], acc[3 * l + d]);
+        if (l == 4) // the row itself: its values lie inside the volume or are zero
+#pragma unroll
+          for (int x = 0; x < 16; x++)
+            accf += fv[x + 1];
       }
     }
   }
 #pragma unroll
   for (int t = 0; t < T; t++)
-    for (int e = 0; e < 4; e++)
-      atomicAdd(dW + (t * C + co) * C + ci0 + e, acc[t][e]);
-  if ((threadIdx.x & 7) == 0)
-    atomicAdd(db + co, accb);
+    red[grp][t][c] = acc[t];
+  red[grp][T][c] = accm;
+  red[grp][T + 1][c] = accf; // the same on every channel
+  __syncthreads();
+  float * dst = part + size_t(blockIdx.x) * kWgIoSums;
+  for (int q = threadIdx.x; q < kWgIoSums; q += 256)
+  {
+    float v = 0.f;
+#pragma unroll
+    for (int g = 0; g < 8; g++)
+      v += red[g][q / C][q % C];
+    dst[q] = v;
+  }
 }
 
-// Layer 1: dW1[t][co] += sum_v dz1[v][co] s x[v + d(t)]; db1[co] += sum_v dz1[v][co].
-// thread: co = tid % 32, tap group tg = tid / 32 (taps tg, tg+8, tg+16, tg+24).
-__global__ __launch_bounds__(256) void wgrad_in_kernel(const float * __restrict__ x, const bf16_t * __restrict__ dz,
-                                                        float * __restrict__ dW, float * __restrict__ db, int B, int X,
-                                                        int Y, int Z, float scale)
+// dst(slot) = sum over the workgroups' slices, in a fixed order: a workgroup takes 64
+// slots, four quarters of the slices, in four chains each.  `where` maps a slot to its
+// place and factor.
+template <class F>
+__device__ __forceinline__ void
+WgReduce(const float * __restrict__ part, int nslots, int nslices, F && where)
 {
-  const int  co = threadIdx.x & 31, tg = threadIdx.x >> 5;
-  const long n = long(B) * X * Y * Z;
-  float      acc[4] = { 0.f, 0.f, 0.f, 0.f }, accb = 0.f;
-  for (long v = blockIdx.x; v < n; v += gridDim.x)
-  {
-    const int   i = int(v % X), j = int((v / X) % Y), k = int((v / (long(X) * Y)) % Z);
-    const float g = float(dz[v * C + co]);
-    if (tg == 0)
-      accb += g;
+  __shared__ float red[4][64];
+  const int slot = blockIdx.x * 64 + (threadIdx.x & 63), quarter = threadIdx.x >> 6;
+  float     v[4] = { 0.f, 0.f, 0.f, 0.f };
+  if (slot < nslots)
+    for (int b = quarter; b < nslices; b += 16)
 #pragma unroll
-    for (int q = 0; q < 4; q++)
-    {
-      const int t = tg + 8 * q;
-      if (t >= T)
-        break;
-      int       dx, dy, dzz;
-      const int off = TapOffset(t, X, Y, dx, dy, dzz);
-      if (i + dx >= 0 && i + dx < X && j + dy >= 0 && j + dy < Y && k + dzz >= 0 && k + dzz < Z)
-        acc[q] += g * scale * x[v + off];
-    }
-  }
-  for (int q = 0; q < 4; q++)
-  {
-    const int t = tg + 8 * q;
-    if (t < T)
-      atomicAdd(dW + t * C + co, acc[q]);
-  }
-  if (tg == 0)
-    atomicAdd(db + co, accb);
+      for (int q = 0; q < 4; q++)
+        if (b + 4 * q < nslices)
+          v[q] += part[size_t(b + 4 * q) * nslots + slot];
+  red[quarter][threadIdx.x & 63] = (v[0] + v[1]) + (v[2] + v[3]);
+  __syncthreads();
+  if (quarter == 0 && slot < nslots)
+    where(slot, (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]));
 }
 
-// Layer 6: dW6[t][ci] += sum_v g[v] a5[v + d(t)][ci]; db6 += sum_v g[v], g = dy / s.
-__global__ __launch_bounds__(256) void wgrad_out_kernel(const bf16_t * __restrict__ a5, const float * __restrict__ dy,
-                                                         float * __restrict__ dW, float * __restrict__ db, int B,
-                                                         int X, int Y, int Z, float inv_scale)
+// 32 -> 32 layer: W and b lie together, in the order of the slots.
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float * __restrict__ part, int nslices,
+                                                            float * __restrict__ g)
 {
-  const int  ci = threadIdx.x & 31, tg = threadIdx.x >> 5;
-  const long n = long(B) * X * Y * Z;
-  float      acc[4] = { 0.f, 0.f, 0.f, 0.f }, accb = 0.f;
-  for (long v = blockIdx.x; v < n; v += gridDim.x)
-  {
-    const int   i = int(v % X), j = int((v / X) % Y), k = int((v / (long(X) * Y)) % Z);
-    const float g = dy[v] * inv_scale;
-    if (threadIdx.x == 0)
-      accb += g;
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-    {
-      const int t = tg + 8 * q;
-      if (t >= T)
-        break;
-      int       dx, dyy, dzz;
-      const int off = TapOffset(t, X, Y, dx, dyy, dzz);
-      if (i + dx >= 0 && i + dx < X && j + dyy >= 0 && j + dyy < Y && k + dzz >= 0 && k + dzz < Z)
-        acc[q] += g * float(a5[(v + off) * C + ci]);
-    }
-  }
-  for (int q = 0; q < 4; q++)
-  {
-    const int t = tg + 8 * q;
+  WgReduce(part, kWgSums, nslices, [&](int slot, float v) { g[slot] = v; });
+}
+
+__global__ __launch_bounds__(256) void wgrad_io_reduce_kernel(const float * __restrict__ part, int nslices,
+                                                               float * __restrict__ g, float factor, int last)
+{
+  WgReduce(part, kWgIoSums, nslices, [&](int slot, float v) {
+    const int t = slot / C, c = slot % C;
     if (t < T)
-      atomicAdd(dW + t * C + ci, acc[q]);
-  }
-  if (threadIdx.x == 0)
-    atomicAdd(db, accb);
+      g[last ? (T - 1 - t) * C + c : slot] = factor * v;
+    else if (last ? slot == kWgIoSums - 1 : t == T)
+      g[T * C + c] = last ? factor * v : v; // db6 (one value), db1 (per channel)
+  });
 }
 
 // ------------------------------------------------------------ loss, Adam, packing
@@ -436,6 +606,7 @@ __global__ void pack_kernel(const float * __restrict__ p, bf16_t * __restrict__ 
 struct rtkhip_cnn
 {
   rtkhip::DeviceBuffer<float>   params, grads, m, v, dy, out;
+  rtkhip::DeviceBuffer<float>   wpart; // per-workgroup sums of the weight gradients (57 MB)
   rtkhip::DeviceBuffer<bf16_t>  wf, wb, act, dz0, dz1;
   rtkhip::DeviceBuffer<double>  partial;
   long                          nvox = 0; // voxels of the activations kept for backward
@@ -492,11 +663,8 @@ ForwardImpl(rtkhip_cnn & net, int B, const int d[3], const float * in, float * o
   net.lastIn = in;
 }
 
-int
-BlocksFor(long n)
-{
-  return int(std::min<long>(std::max<long>(n / 64, 1), 2048));
-}
+// Workgroups of the weight-gradient kernels: two per CU (their LDS), or one a tile.
+constexpr int kWgGroups = 512;
 
 } // namespace
 } // namespace cnn
@@ -604,31 +772,41 @@ rtkhip_cnn_backward(rtkhip_cnn * net, const float * dev_out, const float * dev_t
     float *  P = net->params.get();
     float *  G = net->grads.get();
     bf16_t * A = net->act.get();
-    RTKHIP_CHECK(hipMemsetAsync(G, 0, sizeof(float) * kNumParams, s));
     // loss and dL/dy
     const int gl = int(std::min<long>((n + 255) / 256, 2048));
     hipLaunchKernelGGL(mse_kernel, dim3(gl), dim3(256), 0, s, dev_out, dev_target, net->dy.get(), n, sc * sc,
                        net->partial.get());
     RTKHIP_CHECK_LAUNCH();
     const unsigned g = unsigned((n + 255) / 256);
-    const int      wb = BlocksFor(n);
+    const int  tilesX = (X + 15) / 16, tilesY = (Y + kRowsY - 1) / kRowsY, tilesZ = (Z + 3) / 4;
+    const long nb = long(B) * tilesX * tilesY * tilesZ;
+    const int  ng = int(std::min<long>(nb, kWgGroups));
+    net->wpart.Resize(size_t(ng) * kWgSums);
+    float * part = net->wpart.get();
+    auto    wgradIo = [&](const float * f, const bf16_t * m, float * g, float factor, int last) {
+      hipLaunchKernelGGL(wgrad_io_kernel, dim3(ng), dim3(256), 0, s, f, m, part, X, Y, Z, tilesX, tilesY, tilesZ,
+                         int(nb));
+      RTKHIP_CHECK_LAUNCH();
+      hipLaunchKernelGGL(wgrad_io_reduce_kernel, dim3((kWgIoSums + 63) / 64), dim3(256), 0, s, part, ng, g, factor,
+                         last);
+      RTKHIP_CHECK_LAUNCH();
+    };
     // layer 6
-    hipLaunchKernelGGL(wgrad_out_kernel, dim3(wb), dim3(256), 0, s, A + size_t(4) * n * C, net->dy.get(), G + kL6W,
-                       G + kL6B, B, X, Y, Z, 1.f / sc);
-    RTKHIP_CHECK_LAUNCH();
+    wgradIo(net->dy.get(), A + size_t(4) * n * C, G + kL6W, 1.f / sc, 1);
     hipLaunchKernelGGL(conv_out_bwd_data_kernel, dim3(g), dim3(256), 0, s, net->dy.get(), P, A + size_t(4) * n * C,
                        net->dz0.get(), B, X, Y, Z, 1.f / sc);
     RTKHIP_CHECK_LAUNCH();
     // layers 5..2: dZ_l in dz_cur; weight grads from A_{l-1}; data grad masked by A_{l-1}
-    const int tilesX = (X + 15) / 16, tilesY = (Y + kRowsY - 1) / kRowsY, tilesZ = (Z + 3) / 4;
-    const long nb = long(B) * tilesX * tilesY * tilesZ;
-    bf16_t *   cur = net->dz0.get();
-    bf16_t *   nxt = net->dz1.get();
+    bf16_t * cur = net->dz0.get();
+    bf16_t * nxt = net->dz1.get();
     for (int l = 3; l >= 0; l--) // mid layer index l = layer (l + 2)
     {
       const bf16_t * aprev = A + size_t(l) * n * C; // A_{layer-1} = A[l]
-      hipLaunchKernelGGL(wgrad32_kernel, dim3(wb), dim3(256), 0, s, aprev, cur, G + kMidBase + l * kMidSize,
-                         G + kMidBase + l * kMidSize + T * C * C, B, X, Y, Z);
+      hipLaunchKernelGGL(wgrad32_mfma_kernel, dim3(ng), dim3(256), 0, s, aprev, cur, part, X, Y, Z, tilesX, tilesY,
+                         tilesZ, int(nb));
+      RTKHIP_CHECK_LAUNCH();
+      hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((kWgSums + 63) / 64), dim3(256), 0, s, part, ng,
+                         G + kMidBase + l * kMidSize);
       RTKHIP_CHECK_LAUNCH();
       hipLaunchKernelGGL((conv32_mfma_kernel<false, true>), dim3(unsigned(nb)), dim3(256), 0, s, cur,
                          net->wb.get() + size_t(l) * T * C * C, nullptr, aprev, nxt, X, Y, Z, tilesX, tilesY,
@@ -637,9 +815,7 @@ rtkhip_cnn_backward(rtkhip_cnn * net, const float * dev_out, const float * dev_t
       std::swap(cur, nxt);
     }
     // layer 1 (cur = dZ1)
-    hipLaunchKernelGGL(wgrad_in_kernel, dim3(wb), dim3(256), 0, s, net->lastIn, cur, G + kL1W, G + kL1B, B, X, Y, Z,
-                       sc);
-    RTKHIP_CHECK_LAUNCH();
+    wgradIo(net->lastIn, cur, G + kL1W, sc, 0);
     if (loss)
     {
       std::vector<double> h(gl);

@@ -1,0 +1,50 @@
+"""Weight gradients of the warm-start network on inputs whose arithmetic is exact: small
+integers in every activation, weight and gradient, so BF16 storage and FP32 sums lose
+nothing and the GPU's gradients equal the FP64 oracle's in any order of summation."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _integer_params(rng):
+    """One weight +-1 per output channel (a permutation of the channels at random taps), so
+    activations and data gradients stay within a few units; three per channel in the last
+    layer."""
+    from oracle import cnn_ref
+    C, T = cnn_ref.C, cnn_ref.T
+    d = {"w1": np.zeros((T, C)), "b1": rng.integers(0, 2, C)}
+    d["w1"][rng.integers(0, T, C), np.arange(C)] = rng.choice([1., 1., -1.], C)
+    for l in range(2, 6):
+        w = np.zeros((T, C, C))
+        w[rng.integers(0, T, C), np.arange(C), rng.permutation(C)] = rng.choice([1., 1., 1., -1.], C)
+        d[f"w{l}"], d[f"b{l}"] = w, rng.integers(0, 2, C)
+    d["w6"] = np.zeros((T, C))
+    for _ in range(3):
+        d["w6"][rng.integers(0, T, C), np.arange(C)] = rng.choice([1., -1.], C)
+    d["b6"] = np.ones(1)
+    return cnn_ref.pack(d)
+
+
+# below, at and across the 16 x 4 x 4 tile; batches; more tiles than workgroups (512)
+@pytest.mark.parametrize("shape", [(1, 1, 1, 2), (1, 4, 4, 16), (2, 5, 6, 17), (1, 9, 3, 34), (3, 3, 8, 15),
+                                   (1, 1, 1, 16 * 520 + 2)])
+def test_gradients_are_exact_on_integers(hip, shape):
+    from oracle import cnn_ref
+    from rtk_amd.warmstart import WarmStartCNN
+    rng = np.random.default_rng(sum(shape))
+    p = _integer_params(rng)
+    x = rng.integers(0, 4, shape).astype(np.float32)
+    net = WarmStartCNN(params=p, scale=1.)
+    xd = torch.from_numpy(x).cuda()
+    y = net.forward(xd).cpu().numpy()
+    yr, _ = cnn_ref.forward(p, x.astype(np.float64), 1.)
+    assert np.array_equal(y, yr)
+    # 2 (y - t) / N is a whole number for an even number of voxels N
+    t = (y - rng.integers(-2, 3, shape) * (y.size / 2)).astype(np.float32)
+    loss, _ = net.loss_and_grads(xd, torch.from_numpy(t).cuda())
+    lr, gr = cnn_ref.loss_and_grad(p, x.astype(np.float64), t.astype(np.float64), 1.)
+    assert loss == pytest.approx(lr, rel=1e-12)
+    assert np.any(gr != 0.)
+    assert np.array_equal(net.grads(), gr)
