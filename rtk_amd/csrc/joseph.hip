@@ -84,6 +84,28 @@ __global__ __launch_bounds__(256) void transpose_xz_kernel(const float * __restr
   }
 }
 
+// Copy of the volume with y fastest: out[(z nx + x) pitch + 1 + y], zero for y = -1 and y
+// in [ny, pitch - 1).
+__global__ __launch_bounds__(256) void transpose_xy_kernel(const float * __restrict__ in, float * __restrict__ out,
+                                                            int nx, int ny, int pitch)
+{
+  __shared__ float tile[32][33];
+  const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32, z = blockIdx.z;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5; // 32 x 8
+  for (int r = ty; r < 32; r += 8)
+  {
+    const int x = x0 + tx, y = y0 + r - 1;
+    tile[r][tx] = (x < nx && y >= 0 && y < ny) ? in[(size_t(z) * ny + y) * nx + x] : 0.f;
+  }
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8)
+  {
+    const int y = y0 + tx, x = x0 + r;
+    if (x < nx && y < pitch)
+      out[(size_t(z) * nx + x) * pitch + y] = tile[tx][r];
+  }
+}
+
 // out[z][y][x] += accT[x][y][z]
 __global__ __launch_bounds__(256) void add_transposed_kernel(const float * __restrict__ accT, float * __restrict__ out,
                                                               int nx, int ny, int nz)
@@ -1339,265 +1361,476 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
   vol[idx] += acc;
 }
 
-// Forward projection as a gather, for the geometries the gather backprojection takes
-// (detector columns vertical in the volume).  A column's rays lie in one vertical
-// plane: at slice k of their dominant axis they share the horizontal position X(k),
-// and a middle sample's bilinear interpolation (.hxx:182-543) is the linear
-// interpolation, at the ray's height y'(k), of the profile g(y) = (1 - fx) v(hx, y) +
-// fx v(hx + 1, y) with hx = floor(X), fx = X - hx, the same for every ray of the
-// column.  A workgroup takes 16 columns x kFRows rows of one view; per slice its
-// threads build the 16 profiles over the rows' height range in LDS (double-buffered,
-// one barrier per slice), then each thread adds the middle samples of its kFRays rays
-// (rows 16 apart) from two LDS reads each.  First and last samples, at the ray's own (clamped)
-// positions, read their four taps from global memory as the per-ray projector does.
-// Rays of columns that mix dominant axes are walked per ray.
-constexpr int kFRows = 64; // detector rows per workgroup
-constexpr int kFRays = kFRows / 16; // rays per thread (rows 16 apart)
-constexpr int kFProf = 48; // profile entries per column: kFRows |b| + 3 with |b| < 2/3
-constexpr int kFPad = 49;  // LDS stride of a column's profile (its columns on distinct banks)
-
-// The first and last samples, and every sample of a ray walked alone (a column that
-// mixes dominant axes), as the per-ray forward projector computes them.
-__device__ __forceinline__ float
-RayBorder(const Ray & R, double step, const float * bb, double x, double y)
+// Forward projection of whole detector columns, for the geometries whose detector
+// columns are vertical in the volume.  A column's rays lie in one vertical plane: at slice
+// k of their dominant axis they share the horizontal position X(k), and a middle sample's
+// bilinear interpolation (.hxx:182-543) is the linear interpolation, at the ray's height
+// y'(k) = a(k) + b(k) jv, of the profile g(y) = (1 - fx) v(hx, y) + fx v(hx + 1, y) with
+// hx = floor(X), fx = X - hx, the same for every ray of the column.
+//
+// A wavefront is one column and 64 Q rows of it (lane l: rows l, l + 64, ..), so a slice
+// has one X, and the profile is a run of consecutive heights: in a copy of the volume with
+// y fastest, two contiguous reads of 64 E floats, for slices along x and along z alike.
+// The lanes write the profile to the wavefront's own part of LDS and each ray interpolates
+// two of its values (a wavefront's LDS accesses complete in order: no barrier).  What a
+// slice needs besides (a, b, fx, offsets: FP64 geometry) is computed for 64 slices at once,
+// one slice per lane, and read back from LDS; the runs of the next kBatch slices are in
+// flight while the current ones are summed.  Heights are FP32 relative to the lowest of each
+// group of 64 rows.  Per slice about 20 + 2 E instructions for the profile and 8 per ray, so
+// several rows per lane share one profile.
+// W adjacent columns make a workgroup.  Their runs overlap (X a fraction of a voxel apart),
+// and they are kept within 16 slices of each other by a barrier, so that they share them in
+// L1: without it the wavefronts drift apart and the L2s fetch 264 GB at 512^3 <- 180 x
+// 1024^2 instead of 214 (40 to 48 ms, slower with more wavefronts in flight); the volume
+// read once per view is 97 GB.  Staging the columns' runs in LDS together, a barrier every
+// 2 slices, took 50 ms.  Bound by VALU issue (28 of 37 ms) and the runs' loads together.
+// First and last samples, at the ray's own (clamped) positions, read their four taps.
+// 512^3 -> 180 x 1024^2: 76.5 -> 37.2 ms (before: 16 columns x 64 rows a workgroup, their
+// profiles built and shared in LDS with a barrier every slice); 256^3 -> 360 x 512^2:
+// 18.4 -> 10.6 ms; 64^3 -> one view of 128^2: 55 -> 13 us.
+// A detector column in index coordinates: at slice k its rays are at the horizontal
+// position x0 + k h1 and at the ray parameter t0 + k t1; [near, far] are the slice
+// coordinates between which they cross the volume's horizontal rectangle.
+struct ColumnPath
 {
-  int   tt[4];
-  float w[4];
-  BorderTaps(R, x, y, tt, w);
-  float r = 0.f;
-  r += w[0] * bb[tt[0]];
-  r += w[1] * bb[tt[1]];
-  r += w[2] * bb[tt[2]];
-  r += w[3] * bb[tt[3]];
+  double x0, h1, t0, t1, near, far;
+};
+
+// Narrows [near, far] to where p0 + k slope lies in [0, last].
+__device__ __forceinline__ void
+ClipPath(double p0, double slope, double last, double & near, double & far)
+{
+  if (slope == 0.)
+  {
+    if (!(p0 >= 0. && p0 <= last))
+      far = -1.;
+    return;
+  }
+  const double inv = 1. / slope, a = -p0 * inv, b = (last - p0) * inv;
+  near = fmax(near, fmin(a, b));
+  far = fmin(far, fmax(a, b));
+}
+
+// nk slices, nh horizontal positions.
+__device__ __forceinline__ ColumnPath
+PathOf(const GatherColumn & C, int nk, int nh)
+{
+  const double ck = 0.5 * (nk - 1), ch = 0.5 * (nh - 1);
+  ColumnPath   P{ C.h0 + ch - ck * C.h1, C.h1, C.t0 - ck * C.t1, C.t1, 0., double(nk - 1) };
+  ClipPath(P.x0, P.h1, nh - 1, P.near, P.far);
+  return P;
+}
+
+// One ray of a column: its height y0 + k slope at slice k and the part [near, far] of its
+// path inside the volume.  RTK's first and last samples (.hxx:253-340) are those of the
+// slices round(near) and round(far), weighted by the part of the path within half a slice
+// of them and clamped into the box.
+struct ColumnRay
+{
+  double y0, slope, near, far;
+  __device__ __forceinline__ bool hit() const { return far > near; }
+  __device__ __forceinline__ int  first() const { return int(floor(near + 0.5)); }
+  __device__ __forceinline__ int  last() const { return int(floor(far + 0.5)); }
+};
+__device__ __forceinline__ ColumnRay
+RayOf(const GatherView & V, const ColumnPath & P, int jv, int ny)
+{
+  const double cy = 0.5 * (ny - 1), pix = V.y0 + cy + V.y1 * jv, d = V.sy + cy - pix;
+  ColumnRay    R{ pix + P.t0 * d, P.t1 * d, P.near, P.far };
+  ClipPath(R.y0, R.slope, ny - 1, R.near, R.far);
+  return R;
+}
+
+// Offsets of one step along the in-slice axes (first, second) and along the slices in the
+// y-fastest copy, for a ray of dominant axis `axis`.
+struct ColumnStrides
+{
+  size_t a, b, s;
+};
+__device__ __forceinline__ ColumnStrides
+StridesOf(int axis, int pitch, int nx)
+{
+  const size_t sx = pitch, sz = size_t(pitch) * nx;
+  return axis == 0 ? ColumnStrides{ sz, 1, sx } : (axis == 1 ? ColumnStrides{ sx, sz, 1 } : ColumnStrides{ sx, 1, sz });
+}
+
+// The first or last sample of a column's ray, at slice k, weighted by `step`
+// (BilinearInterpolationOnBorders, .hxx:493-543: taps outside the box are clamped inward).
+__device__ __forceinline__ float
+EndSample(const ColumnPath & P, const ColumnRay & R, int k, double step, const float * vol, const ColumnStrides & S,
+          int nh, int ny)
+{
+  const double x = P.x0 + k * P.h1, y = R.y0 + k * R.slope;
+  const int    ix = min(max(int(floor(x)), -1), nh - 1), iy = min(max(int(floor(y)), -1), ny - 1);
+  const double lx = x - ix, ly = y - iy, lxc = 1. - lx, lyc = 1. - ly;
+  const int    xa = max(ix, 0), xb = ix + 1 - (ix >= nh - 1 ? 1 : 0);
+  const int    ya = max(iy, 0), yb = iy + 1 - (iy >= ny - 1 ? 1 : 0);
+  const float *va = vol + k * S.s + xa * S.a, *vb = vol + k * S.s + xb * S.a;
+  float        r = 0.f;
+  r += float(lxc * lyc) * va[ya];
+  r += float(lxc * ly) * va[yb];
+  r += float(lx * lyc) * vb[ya];
+  r += float(lx * ly) * vb[yb];
   return float(double(r) * step);
 }
 
+// Rays of the columns the sweep does not take (they mix dominant axes, or lie so close to
+// a change of axis that rounding decides it), one ray per thread, as the per-ray forward
+// projector walks them.  columns: view * nu + iu.
 __device__ __forceinline__ float
-RayEnds(const Ray & R, const float * vol, const float * volT)
+RayBorder(const Ray & R, const ColumnStrides & S, double step, const float * slice, double x, double y)
 {
-  const float * b = (R.transposed ? volT : vol) + R.start;
-  if (R.fs == R.ns)
-    return RayBorder(R, R.wOne, b, R.cx, R.cy);
-  const float first = RayBorder(R, R.wB, b, R.cx, R.cy);
-  const double n = double(R.nmid + 1);
-  return first + RayBorder(R, R.wE, b + (R.nmid + 1) * R.oz, R.cx + n * R.stepx, R.cy + n * R.stepy);
+  int   tx[4], ty[4];
+  float w[4];
+  BorderTaps2D(R, x, y, tx, ty, w);
+  float r = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    r += w[q] * slice[size_t(tx[q]) * S.a + size_t(ty[q]) * S.b];
+  return float(double(r) * step);
 }
+
+__global__ __launch_bounds__(64) void joseph_fp_single_kernel(const JosephView * __restrict__ views,
+                                                               const int * __restrict__ columns, int nu, int nv,
+                                                               const float * pin, float * pout,
+                                                               const float * __restrict__ vol, int pitch, int nx,
+                                                               int ny, int nz, double spx, double spy, double spz,
+                                                               double infClip, double supClip)
+{
+  const int p = columns[blockIdx.x] / nu, iu = columns[blockIdx.x] % nu, jv = blockIdx.y * 64 + threadIdx.x;
+  if (jv >= nv)
+    return;
+  const size_t pix = (size_t(p) * nv + jv) * nu + iu;
+  const float  base = pin ? pin[pix] : 0.f;
+  Ray          R;
+  if (!SetupRay<false>(views[p], iu, jv, p, nx, ny, nz, spx, spy, spz, infClip, supClip, R))
+  {
+    pout[pix] = base;
+    return;
+  }
+  const ColumnStrides S = StridesOf(R.axis, pitch, nx);
+  float               sum;
+  if (R.fs == R.ns)
+    sum = RayBorder(R, S, R.wOne, vol + R.ns * S.s, R.cx, R.cy);
+  else
+  {
+    sum = RayBorder(R, S, R.wB, vol + R.ns * S.s, R.cx, R.cy);
+    const int dir = R.fs > R.ns ? 1 : -1;
+    Walker    wk;
+    wk.Init(R.cx + R.stepx, R.cy + R.stepy);
+    for (int k = R.ns + dir; k != R.fs; k += dir)
+    {
+      int   cx, cy;
+      float lx, ly;
+      wk.Stage2D(R, cx, cy, lx, ly);
+      const float * b = vol + k * S.s + cx * S.a + cy * S.b;
+      const float   lxc = 1.f - lx, lyc = 1.f - ly;
+      sum += (lxc * lyc) * b[0] + (lx * lyc) * b[S.a] + (lxc * ly) * b[S.b] + (lx * ly) * b[S.a + S.b];
+    }
+    sum += RayBorder(R, S, R.wE, vol + R.fs * S.s, wk.PosX(), wk.PosY());
+  }
+  pout[pix] = float(double(base) + double(sum) * R.stepNorm);
+}
+
+template <int E>
+struct ProfileRuns
+{
+  float v0[E], v1[E]; // this lane's heights of the runs at hx and hx + 1
+};
 
 __device__ __forceinline__ float
-RayWalk(const Ray & R, const float * vol, const float * volT)
+ReadLane(float v, int lane)
 {
-  const float * b = (R.transposed ? volT : vol) + R.start;
-  if (R.fs == R.ns)
-    return RayBorder(R, R.wOne, b, R.cx, R.cy);
-  float sum = RayBorder(R, R.wB, b, R.cx, R.cy);
-  b += R.oz;
-  Walker wk;
-  wk.Init(R.cx + R.stepx, R.cy + R.stepy);
-  for (int s2 = 0; s2 < R.nmid; ++s2)
-  {
-    float       lx, ly;
-    const int   idx = wk.Stage(R, lx, ly);
-    const float lxc = 1.f - lx, lyc = 1.f - ly;
-    sum += (lxc * lyc) * b[idx] + (lx * lyc) * b[idx + 1] + (lxc * ly) * b[idx + R.oy] + (lx * ly) * b[idx + 1 + R.oy];
-    b += R.oz;
-  }
-  return sum + RayBorder(R, R.wE, b, wk.PosX(), wk.PosY());
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// Middle samples of the columns of dominant axis A (0: slices along x in the z-fastest
-// copy, horizontal z; 2: slices along z, horizontal x), slices klo..khi (uniform over
-// the workgroup).  Ray q of this thread takes the slices lo[q]..hi[q].  The profile
-// values of slice k + 1 are loaded while the rays of slice k are summed.
-template <int A>
-__device__ __forceinline__ void
-ForwardGatherSweep(const GatherView & V, const GatherColumn & C, bool colOn, const int (&lo)[kFRays], const int (&hi)[kFRays],
-                   int jv0, int rb, int rlast, const float * __restrict__ buf, int nsl, int nh, int ny, int klo,
-                   int khi, float (*prof)[16][kFPad], float (&acc)[kFRays])
+template <int W, int Q, int E>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(Q <= 2 ? 7 : 6))) void joseph_fp_column_kernel(
+  const GatherView * __restrict__ gviews, const GatherColumn * __restrict__ gcols,
+  const signed char * __restrict__ colAxis, int nu, int nv, const float * pin, float * pout,
+  const float * __restrict__ vol, int pitch, int nx, int ny, int nz, double spx, double spy, double spz,
+  int xcdOrder)
 {
-  const int    t = threadIdx.x, c = t & 15, rq = t >> 4;
-  const size_t sk = size_t(ny) * nh; // slice stride; rows nh apart, the horizontal axis unit-stride
-  const double ck = 0.5 * (nsl - 1), ch = 0.5 * (nh - 1), cy = 0.5 * (ny - 1);
-  constexpr int NM = kFProf / 16; // profile entries per thread
-  // the column at slice k: the rows' heights a + b jv relative to the profile's first
-  // height ylo (Af + Bf jv), and this thread's profile entries as tap pairs
-  struct Slice
-  {
-    float  Af, Bf, fx;
-    int    ylo;
-    float2 v[NM];
-  };
-  // X and t advance by h1 and t1 per slice; a and b are affine in t
-  const double kd0 = double(klo) - ck;
-  double       X = C.h0 + kd0 * C.h1 + ch, tt = C.t0 + kd0 * C.t1;
-  const double dsy = V.sy - V.y0, a0 = V.y0 + cy;
-  auto         fetch = [&](int k, Slice & S) {
-    if (!colOn || k > khi)
-      return;
-    const double a = fma(tt, dsy, a0), b = fma(-V.y1, tt, V.y1);
-    const double fl = floor(X);
-    const int    hx = min(max(int(fl), 0), nh - 2);
-    S.fx = float(X - fl);
-    S.ylo = int(floor(fmin(a + b * rb, a + b * rlast)));
-    S.Af = float(a - double(S.ylo));
-    S.Bf = float(b);
-    // entries rq + 16 m: heights ylo + rq + 16 m (zero outside the volume)
-    const int     y0 = S.ylo + rq;
-    const float * q0 = buf + (size_t(k) * sk + hx) + ptrdiff_t(y0) * nh;
-#pragma unroll
-    for (int m = 0; m < NM; m++)
-    {
-      const float * q = q0 + 16 * m * nh;
-      S.v[m] = unsigned(y0 + 16 * m) < unsigned(ny) ? make_float2(q[0], q[1]) : make_float2(0.f, 0.f);
-    }
-    X += C.h1;
-    tt += C.t1;
-  };
-  Slice cur{}, nxt{};
-  fetch(klo, cur);
-  for (int k = klo; k <= khi; k++)
-  {
-    float(*g)[kFPad] = prof[k & 1];
-    if (colOn)
-    {
-#pragma unroll
-      for (int m = 0; m < NM; m++)
-        g[c][rq + 16 * m] = (1.f - cur.fx) * cur.v[m].x + cur.fx * cur.v[m].y;
-    }
-    __syncthreads();
-    fetch(k + 1, nxt);
-    if (colOn)
-    {
-#pragma unroll
-      for (int q = 0; q < kFRays; q++)
-      {
-        if (k < lo[q] || k > hi[q])
-          continue;
-        // the row pair of the ray's height, its index clamped as the per-ray walk
-        // clamps it, the fraction unclamped
-        // (entries outside the volume are zero; the index bound only guards rounding)
-        const float u = fmaxf(fmaf(cur.Bf, float(jv0 + 16 * q), cur.Af), 0.f); // y' - ylo (>= 0 but for rounding)
-        const float fu = floorf(u);
-        const float fy = u - fu;
-        const int   iy = min(int(fu), kFProf - 2);
-        const float g0 = g[c][iy];
-        acc[q] += fmaf(fy, g[c][iy + 1] - g0, g0);
-      }
-    }
-    cur = nxt;
-  }
-  __syncthreads();
-}
-
-__global__ __launch_bounds__(256) void joseph_fp_gather_kernel(
-  const JosephView * __restrict__ views, const GatherView * __restrict__ gviews,
-  const GatherColumn * __restrict__ gcols, const signed char * __restrict__ colAxis, int nu, int nv,
-  const float * pin, float * pout, const float * __restrict__ vol, const float * __restrict__ volT, int nx, int ny,
-  int nz, double spx, double spy, double spz, double infClip, double supClip, int xcdOrder)
-{
-  __shared__ float prof[2][16][kFPad];
-  __shared__ int   krange[2][2]; // [x / z columns][first, last middle slice]
-  const int        t = threadIdx.x, c = t & 15, rq = t >> 4;
-  // grid (column blocks, views, row bands), as the per-ray projector: workgroups in
-  // flight share a band of detector rows, whose rays stay in one slab of the volume,
-  // so the slab stays in L2 while every view reads it
-  // Workgroups are dealt to the 8 XCDs in turn in linear order.  xcdOrder 1 renumbers
-  // them so that XCD x takes a contiguous run of (column block, view, row band)
-  // triples: its L2 then serves one band's rays, and the 8 XCDs read 8 bands' slabs of
-  // the volume at once (for volumes whose two copies fit the last-level cache).
-  // xcdOrder 2 keeps the bands in order and, within a band, gives XCD x a contiguous
-  // run of its (column block, view) pairs: all XCDs read one slab, each for a range of
-  // neighbouring views.
-  const unsigned   nblk = gridDim.x * gridDim.y * gridDim.z, full = nblk / 8, rem = nblk % 8;
-  const unsigned   lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  unsigned         blk = lin;
+  constexpr int    kSync = 16; // slices between barriers
+  constexpr int    kBatch = E >= 3 ? 2 : 4; // slices whose runs are loaded together
+  constexpr int    GW = Q <= 2 ? 4 : 8; // per slice: the groups' a, then b and fx
+  __shared__ float  prof[W][kBatch * 64 * E];
+  __shared__ float  geom[W][64][GW];
+  __shared__ int    krange[2];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Grid (column blocks, views, row bands): workgroups in flight share a band of detector
+  // rows, whose rays stay in one slab of the volume.  Workgroups are dealt to the 8 XCDs
+  // in turn in linear order; xcdOrder 1 renumbers them so that each XCD takes a contiguous
+  // run of (column block, view, band) triples, xcdOrder 2 so that within each band, all
+  // XCDs in the same one, each takes a contiguous run of its (column block, view) pairs.
+  const unsigned nblk = gridDim.x * gridDim.y * gridDim.z, full = nblk / 8, rem = nblk % 8;
+  const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  unsigned       blk = lin;
   if (xcdOrder == 1)
     blk = (lin % 8) * full + min(lin % 8, rem) + lin / 8;
   else if (xcdOrder == 2)
   {
-    // within each row band: XCD x takes a contiguous run of its (column block, view) pairs
     const unsigned P = gridDim.x * gridDim.y, w = lin % P, f = P / 8, r = P % 8, x = w % 8;
     blk = (lin / P) * P + x * f + min(x, r) + w / 8;
   }
-  const int        p = int((blk / gridDim.x) % gridDim.y), iu = int(blk % gridDim.x) * 16 + c,
-                   rb = int(blk / (gridDim.x * gridDim.y)) * kFRows;
-  const int        rlast = min(rb + kFRows, nv) - 1;
-  const int        jv0 = rb + rq; // this thread's rays: rows jv0 + 16 q
-  if (t < 2)
-  {
-    krange[t][0] = INT_MAX;
-    krange[t][1] = INT_MIN;
-  }
-  __syncthreads();
+  const int p = int((blk / gridDim.x) % gridDim.y), u0 = int(blk % gridDim.x) * W, iu = u0 + wave,
+            r0 = int(blk / (gridDim.x * gridDim.y)) * (64 * Q);
+  // whether the workgroup's columns all walk along one axis, and so keep together
   const int cax = iu < nu ? int(colAxis[size_t(p) * nu + iu]) : -1;
-  float     acc[kFRays];
-  double    norm[kFRays];
-  int       lo[kFRays], hi[kFRays];
-  bool      hit[kFRays];
-  int       klo = INT_MAX, khi = INT_MIN;
+  bool      together = u0 + W <= nu && cax >= 0;
+  for (int c = 0; c < W && together; c++)
+    together = int(colAxis[size_t(p) * nu + u0 + c]) == cax;
+  if (cax < 0) // beyond the detector, or joseph_fp_single_kernel's
+    return;
+  const int rlast = min(r0 + 64 * Q, nv) - 1;
+  const bool          alongX = cax == 0;
+  const int           nk = alongX ? nx : nz, nh = alongX ? nz : nx;
+  const ColumnStrides S = StridesOf(cax, pitch, nx);
+  const GatherView &  V = gviews[p];
+  const GatherColumn  C = gcols[size_t(p) * nu + iu];
+  const ColumnPath    P = PathOf(C, nk, nh);
+  // A ray's first and last samples, and the middle slices of a ray that has any as first |
+  // last << 16 (else 1: first above last).  Only what the sweep needs is kept: the rest is
+  // computed again after it, which leaves the registers to the loads in flight.
+  auto endsOf = [&](const ColumnRay & R) {
+    const int ns = R.first(), fs = R.last();
+    return ns == fs ? EndSample(P, R, ns, R.far - R.near, vol, S, nh, ny)
+                    : EndSample(P, R, ns, ns + 0.5 - R.near, vol, S, nh, ny) +
+                        EndSample(P, R, fs, R.far - (fs - 0.5), vol, S, nh, ny);
+  };
+  float    acc[Q];
+  unsigned middle[Q];
 #pragma unroll
-  for (int q = 0; q < kFRays; q++)
+  for (int q = 0; q < Q; q++)
   {
-    const int jv = jv0 + 16 * q;
-    Ray       R;
+    const int       jv = r0 + lane + 64 * q;
+    const ColumnRay R = RayOf(V, P, jv, ny);
     acc[q] = 0.f;
-    norm[q] = 0.;
-    hit[q] = iu < nu && jv < nv && SetupRay<false>(views[p], iu, jv, p, nx, ny, nz, spx, spy, spz, infClip, supClip, R);
-    lo[q] = 1;
-    hi[q] = 0;
-    if (!hit[q])
-      continue;
-    norm[q] = R.stepNorm;
-    if (cax < 0 || R.axis != cax)
-      acc[q] = RayWalk(R, vol, volT); // a column that mixes dominant axes
-    else
+    middle[q] = 1u;
+    if (jv < nv && R.hit() && R.first() + 1 < R.last())
     {
-      acc[q] = RayEnds(R, vol, volT);
-      lo[q] = min(R.ns, R.fs) + 1; // middle slices
-      hi[q] = max(R.ns, R.fs) - 1;
-      klo = min(klo, lo[q]);
-      khi = max(khi, hi[q]);
+      acc[q] = endsOf(R);
+      middle[q] = unsigned(R.first() + 1) | unsigned(R.last() - 1) << 16;
     }
   }
-  if (cax >= 0 && klo <= khi)
-  {
-    atomicMin(&krange[cax >> 1][0], klo);
-    atomicMax(&krange[cax >> 1][1], khi);
-  }
-  __syncthreads();
-  const GatherView V = gviews[p];
-  GatherColumn     C{};
-  if (cax >= 0)
-    C = gcols[size_t(p) * nu + iu];
-  if (krange[0][0] <= krange[0][1])
-    ForwardGatherSweep<0>(V, C, cax == 0, lo, hi, jv0, rb, rlast, volT, nx, nz, ny, krange[0][0], krange[0][1], prof,
-                          acc);
-  if (krange[1][0] <= krange[1][1])
-    ForwardGatherSweep<2>(V, C, cax == 2, lo, hi, jv0, rb, rlast, vol, nz, nx, ny, krange[1][0], krange[1][1], prof,
-                          acc);
+  auto lo = [&](int q) { return int(middle[q] & 0xffffu); };
+  auto hi = [&](int q) { return int(middle[q] >> 16); };
+  // slices some ray of the wavefront samples, and slices all of them do (the rays without a
+  // middle sample apart)
+  int wlo = INT_MAX, whi = INT_MIN, wall = INT_MIN, wend = INT_MAX;
 #pragma unroll
-  for (int q = 0; q < kFRays; q++)
+  for (int q = 0; q < Q; q++)
+    if (lo(q) <= hi(q))
+    {
+      wlo = min(wlo, lo(q));
+      whi = max(whi, hi(q));
+      wall = max(wall, lo(q));
+      wend = min(wend, hi(q));
+    }
+  for (int o = 32; o > 0; o >>= 1)
   {
-    const int jv = jv0 + 16 * q;
-    if (iu >= nu || jv >= nv)
+    wlo = min(wlo, __shfl_xor(wlo, o, 64));
+    whi = max(whi, __shfl_xor(whi, o, 64));
+    wall = max(wall, __shfl_xor(wall, o, 64));
+    wend = min(wend, __shfl_xor(wend, o, 64));
+  }
+  wlo = __builtin_amdgcn_readfirstlane(wlo);
+  whi = __builtin_amdgcn_readfirstlane(whi);
+  wall = __builtin_amdgcn_readfirstlane(wall);
+  wend = __builtin_amdgcn_readfirstlane(wend);
+  if (wlo > whi)
+    wall = INT_MAX; // no ray in the sweep
+  if (together)
+  {
+    if (threadIdx.x < 2)
+      krange[threadIdx.x] = threadIdx.x ? INT_MIN : INT_MAX;
+    __syncthreads();
+    if (lane == 0)
+    {
+      atomicMin(&krange[0], wlo);
+      atomicMax(&krange[1], whi);
+    }
+    __syncthreads();
+    wlo = __builtin_amdgcn_readfirstlane(krange[0]);
+    whi = __builtin_amdgcn_readfirstlane(krange[1]);
+  }
+  if (wlo <= whi)
+  {
+    const unsigned sk = unsigned(S.s), sh = unsigned(S.a);
+    const double   cy = 0.5 * (ny - 1);
+    float *        mine = prof[wave];
+    // The rays' rows.  A lane without a ray in the sweep repeats one of its group that has,
+    // a group without one repeats a group that has, so that their (unused) sums read
+    // inside the profile too.
+    float rowf[Q];
+    int   some[Q], group[Q], any = 0;
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+    {
+      const unsigned long long m = __ballot(lo(q) <= hi(q));
+      some[q] = m ? r0 + 64 * q + __ffsll(m) - 1 : -1;
+      any = m ? q : any;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+    {
+      int r = some[q];
+      group[q] = q;
+#pragma unroll
+      for (int o = 0; o < Q; o++)
+        if (some[q] < 0 && o == any)
+        {
+          r = some[o];
+          group[q] = o;
+        }
+      rowf[q] = float(lo(q) <= hi(q) ? r0 + lane + 64 * q : r);
+    }
+    for (int kc = wlo; kc <= whi; kc += 64)
+    {
+      // the column at slice kc + lane: heights relative to the run's first one
+      const double   kd = double(kc + lane);
+      const double   X = P.x0 + kd * P.h1, tt = P.t0 + kd * P.t1;
+      const double   a = fma(tt, V.sy - V.y0, V.y0 + cy), b = fma(-V.y1, tt, V.y1);
+      const double   ya = a + b * r0, yb = a + b * rlast, fl = floor(X);
+      const int      hx = min(max(int(fl), 0), nh - 2);
+      // the run of 64 E heights from ylo, one below the band's lowest (a height rounded below
+      // the volume reads the zero there), holds every height of the band in the volume
+      const int      ylo = min(max(int(floor(fmin(ya, yb))), 0) - 1, pitch - 1 - 64 * E);
+      // each group of 64 rows takes its heights relative to its own lowest, so their FP32
+      // values stay small; rel: that height in the run, 16 bits a group
+      unsigned rel[2] = { 0, 0 };
+      auto *   gl = geom[wave][lane];
+#pragma unroll
+      for (int q = 0; q < Q; q++)
+      {
+        const int    rb = r0 + 64 * group[q], re = min(rb + 64, nv) - 1;
+        const double al = a + b * rb, ah = a + b * re;
+        const int    yq = int(floor(fmin(al, ah)));
+        gl[q] = float(a - double(yq));
+        rel[q >> 1] |= unsigned((yq - ylo) & 0xffff) << (16 * (q & 1));
+      }
+      gl[GW - 2] = float(b);
+      gl[GW - 1] = float(X - fl);
+      __builtin_amdgcn_wave_barrier();
+      const unsigned offl = unsigned(kc + lane) * sk + unsigned(hx) * sh + unsigned(ylo + 1);
+      const int      n = min(64, whi - kc + 1);
+      // the runs of kBatch slices from slice kk of the chunk (the last one again beyond it)
+      auto fetch = [&](int kk, ProfileRuns<E>(&r)[kBatch]) {
+#pragma unroll
+        for (int j = 0; j < kBatch; j++)
+        {
+          const unsigned off = unsigned(__builtin_amdgcn_readlane(int(offl), min(kk + j, n - 1)));
+          const float *  b0 = vol - 1 + size_t(off), * b1 = b0 + sh;
+#pragma unroll
+          for (int e = 0; e < E; e++)
+          {
+            r[j].v0[e] = b0[lane + 64 * e];
+            r[j].v1[e] = b1[lane + 64 * e];
+          }
+        }
+      };
+      // their profiles to LDS, then the samples
+      auto sum = [&](int kk, const ProfileRuns<E>(&r)[kBatch]) {
+        if (kk >= n)
+          return;
+        float A[kBatch][Q], B[kBatch];
+        int   base[kBatch][Q];
+#pragma unroll
+        for (int j = 0; j < kBatch; j++)
+        {
+          const int     at = min(kk + j, n - 1);
+          const float * gs = geom[wave][at];
+          const float   fx = gs[GW - 1], fc = 1.f - fx;
+#pragma unroll
+          for (int e = 0; e < E; e++)
+            mine[j * 64 * E + lane + 64 * e] = fmaf(fc, r[j].v0[e], fx * r[j].v1[e]);
+          B[j] = gs[GW - 2];
+          const int o[2] = { __builtin_amdgcn_readlane(int(rel[0]), at),
+                             Q > 2 ? __builtin_amdgcn_readlane(int(rel[1]), at) : 0 };
+#pragma unroll
+          for (int q = 0; q < Q; q++)
+          {
+            A[j][q] = gs[q];
+            base[j][q] = j * 64 * E + ((q & 1) ? o[q >> 1] >> 16 : int(short(o[q >> 1] & 0xffff)));
+          }
+        }
+        const int k0 = kc + kk, k1 = k0 + kBatch - 1;
+        if (kk + kBatch <= n && k0 >= wall && k1 <= wend)
+        {
+          // every ray samples every one of these slices
+#pragma unroll
+          for (int j = 0; j < kBatch; j++)
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+            {
+              const float   u = fmaxf(fmaf(B[j], rowf[q], A[j][q]), 0.f), fy = __builtin_amdgcn_fractf(u);
+              const float * g = mine + (base[j][q] + int(u));
+              acc[q] += fmaf(fy, g[1] - g[0], g[0]);
+            }
+          return;
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; j++)
+#pragma unroll
+          for (int q = 0; q < Q; q++)
+          {
+            const float   u = fmaxf(fmaf(B[j], rowf[q], A[j][q]), 0.f), fy = __builtin_amdgcn_fractf(u);
+            // rays outside the volume at this slice read any height of the run
+            const float * g = mine + min(max(base[j][q] + int(fminf(u, 512.f)), j * 64 * E), (j + 1) * 64 * E - 2);
+            float         s = fmaf(fy, g[1] - g[0], g[0]);
+            // opaque to the optimiser: a select, not a branch around the LDS reads
+            __asm__("" : "+v"(s));
+            acc[q] += (kk + j < n && k0 + j >= lo(q) && k0 + j <= hi(q)) ? s : 0.f;
+          }
+      };
+      // two sets of registers in turn: one set's loads are in flight while the other's
+      // samples are summed
+      ProfileRuns<E> even[kBatch], odd[kBatch];
+      fetch(0, even);
+#pragma unroll 1
+      for (int kk = 0; kk < n; kk += 2 * kBatch)
+      {
+        if (together && kk % kSync == 0)
+          __syncthreads();
+        fetch(kk + kBatch, odd);
+        sum(kk, even);
+        fetch(kk + 2 * kBatch, even);
+        sum(kk + kBatch, odd);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+  {
+    const int jv = r0 + lane + 64 * q;
+    if (jv >= nv)
       continue;
-    const long pix = (long(p) * nv + jv) * nu + iu;
-    if (hit[q])
-      pout[pix] = float(double(pin ? pin[pix] : 0.f) + double(acc[q]) * norm[q]);
-    else
-      pout[pix] = pin ? pin[pix] : 0.f;
+    const ColumnRay R = RayOf(V, P, jv, ny);
+    const size_t    pix = (size_t(p) * nv + jv) * nu + iu;
+    const float     base = pin ? pin[pix] : 0.f;
+    if (!R.hit())
+    {
+      pout[pix] = base;
+      continue;
+    }
+    // a ray without a middle sample took no part in the sweep
+    const float  sum = R.first() + 1 < R.last() ? acc[q] : endsOf(R);
+    const double stepy = spy * R.slope, steph = (alongX ? spz : spx) * P.h1, stepk = alongX ? spx : spz;
+    pout[pix] = float(double(base) + double(sum) * sqrt(steph * steph + stepy * stepy + stepk * stepk));
   }
 }
 
 struct JosephCache
 {
   std::map<hipStream_t, DeviceBuffer<JosephView>>          views;
-  std::map<hipStream_t, DeviceBuffer<float>>               volT;
+  std::map<hipStream_t, DeviceBuffer<float>>               volT; // z- or y-fastest copy of the volume
   std::map<hipStream_t, DeviceBuffer<unsigned long long>> count;
   // gather backprojection: per-view and per-column tables, block lists, per-ray data
   std::map<hipStream_t, DeviceBuffer<GatherView>>   gviews;
   std::map<hipStream_t, DeviceBuffer<GatherColumn>> gcols;
   std::map<hipStream_t, DeviceBuffer<signed char>>  gaxis;
   std::map<hipStream_t, DeviceBuffer<int>>          gblocks;
+  std::map<hipStream_t, DeviceBuffer<int>>          gsingle;
   std::map<hipStream_t, DeviceBuffer<float>>        gval;
   std::map<hipStream_t, DeviceBuffer<uint2>>        gend;
   std::map<hipStream_t, DeviceBuffer<float2>>       gw;
@@ -1610,7 +1843,8 @@ struct JosephCache
   std::map<hipStream_t, std::vector<double>> gplanKey;
   std::map<hipStream_t, long long>           gplanBlocks; // -1: the gather does not apply
   std::map<hipStream_t, int>                 gplanFree;
-  std::map<hipStream_t, bool>                gplanForward;
+  std::map<hipStream_t, int>                        gplanSingle; // entries of gsingle
+  std::map<hipStream_t, double>                     gplanRowStep;
 };
 thread_local JosephCache g_joseph;
 
@@ -1620,9 +1854,10 @@ struct GatherPlan
   std::vector<GatherView>   views;
   std::vector<GatherColumn> cols;
   std::vector<signed char>  axis;
+  std::vector<int>          single; // columns (view * nu + iu) of no single axis, taken ray by ray
   std::vector<int>          blocks; // packed block coordinates (bx | bz << 10 | by << 20)
   int                       freeRows = 1; // leading candidate rows whose weight needs no clamp
-  bool                      forward = false; // the forward gather's profiles hold kFRows rows
+  double                    maxRowStep = 0.; // largest height step between adjacent rows inside the volume
 };
 
 // True when the geometry lets the gather take the backprojection: default clips,
@@ -1691,13 +1926,18 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
     {
       const double px = o[0] + iu * eu[0], pz = o[2] + iu * eu[2];
       const double dx = S[0] - px, dz = S[2] - pz;
-      int          ax = -1;
-      if (std::abs(dx) >= std::abs(dz) && std::abs(dx) >= mh)
+      // a margin keeps the columns whose dominant axis rounding decides out of the tables
+      constexpr double kTie = 1. + 1e-9;
+      int              ax = -1;
+      if (std::abs(dx) > kTie * std::abs(dz) && std::abs(dx) > kTie * mh)
         ax = 0;
-      else if (std::abs(dz) > std::abs(dx) && std::abs(dz) > mh)
+      else if (std::abs(dz) > kTie * std::abs(dx) && std::abs(dz) > kTie * mh)
         ax = 2;
       if (ax < 0)
+      {
+        G.single.push_back(p * nu + iu);
         continue;
+      }
       GatherColumn & C = G.cols[size_t(p) * nu + iu];
       const double   dk = ax == 0 ? dx : dz, dh = ax == 0 ? dz : dx;
       const double   pk = ax == 0 ? px : pz, ph = ax == 0 ? pz : px;
@@ -1743,9 +1983,7 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
   // the first candidate row has |y' - j| < 1 and rows advance by the step b, so rows
   // 0..2 stay inside the window when 3 |b| < 2 (a margin covers the FP32 arithmetic)
   G.freeRows = maxRowStep < (2. / 3.) * (1. - 1e-4) ? 3 : 1;
-  // kFRows rows span (kFRows - 1) |b| + 1 heights above the profile's first one, and
-  // a middle sample reads two entries
-  G.forward = maxRowStep * (kFRows - 1) * (1. + 1e-4) + 3. <= double(kFProf);
+  G.maxRowStep = maxRowStep;
   const int nbx = (nx + 15) / 16, nbz = (nz + 15) / 16, nby = (ny + kGNJ - 1) / kGNJ;
   G.blocks.clear();
   for (int by = 0; by < nby; by++)
@@ -1764,7 +2002,7 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
 // of gather blocks, or -1 when the gather does not apply.
 long long
 PrepareGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vol, const double * source,
-              double inferior_clip, double superior_clip, hipStream_t s, int & freeRows, bool * forward = nullptr)
+              double inferior_clip, double superior_clip, hipStream_t s, int & freeRows, double * maxRowStep = nullptr)
 {
   const int           np = proj_dim[2], nu = proj_dim[0];
   std::vector<double> key = { double(proj_dim[0]), double(proj_dim[1]), double(np),           double(vol_dim[0]),
@@ -1778,8 +2016,8 @@ PrepareGather(const int proj_dim[3], const int vol_dim[3], const double * proj_t
   if (cached == key)
   {
     freeRows = g_joseph.gplanFree[s];
-    if (forward)
-      *forward = g_joseph.gplanForward[s];
+    if (maxRowStep)
+      *maxRowStep = g_joseph.gplanRowStep[s];
     return g_joseph.gplanBlocks[s];
   }
   cached.clear(); // a failure below leaves no stale entry
@@ -1801,13 +2039,21 @@ PrepareGather(const int proj_dim[3], const int vol_dim[3], const double * proj_t
     RTKHIP_CHECK(hipMemcpyAsync(ga.get(), G.axis.data(), G.axis.size(), hipMemcpyHostToDevice, s));
     RTKHIP_CHECK(
       hipMemcpyAsync(gb.get(), G.blocks.data(), sizeof(int) * G.blocks.size(), hipMemcpyHostToDevice, s));
+    if (!G.single.empty())
+    {
+      auto & gs = g_joseph.gsingle[s];
+      gs.Resize(G.single.size());
+      RTKHIP_CHECK(
+        hipMemcpyAsync(gs.get(), G.single.data(), sizeof(int) * G.single.size(), hipMemcpyHostToDevice, s));
+    }
     nblocks = (long long)G.blocks.size();
   }
+  g_joseph.gplanSingle[s] = int(G.single.size());
   g_joseph.gplanBlocks[s] = nblocks;
   g_joseph.gplanFree[s] = freeRows = G.freeRows;
-  g_joseph.gplanForward[s] = nblocks >= 0 && G.forward;
-  if (forward)
-    *forward = g_joseph.gplanForward[s];
+  g_joseph.gplanRowStep[s] = G.maxRowStep;
+  if (maxRowStep)
+    *maxRowStep = G.maxRowStep;
   cached = std::move(key);
   return nblocks;
 }
@@ -1898,6 +2144,44 @@ CheckArgs(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vo
   RTKHIP_REQUIRE(nvox < (1LL << 31), RTKHIP_ERR_UNSUPPORTED, "joseph: volumes are limited to 2^31 voxels");
 }
 
+// Columns a workgroup (W), rows per lane (Q) and profile heights per lane (E) of
+// joseph_fp_column_kernel: the candidates whose 64 E heights hold 64 Q rows at the geometry's largest row step and four
+// heights for the floor and the neighbours above and below.
+struct ColumnShape
+{
+  int w = 0, q = 0, e = 0;
+};
+#define RTKHIP_COLUMN_SHAPES(X)                                                                                      \
+  X(4, 1, 1) X(4, 1, 2) X(8, 1, 2) X(8, 2, 2) X(8, 2, 3) X(8, 3, 2) X(8, 3, 3) X(8, 3, 4) X(8, 4, 3) X(8, 4, 4)
+ColumnShape
+ChooseColumnShape(double maxRowStep, int nu, int nv, int np)
+{
+  // Larger steps keep the per-ray kernel: fewer than 1.4 rows a voxel share a profile, and
+  // that kernel's sums round the positions otherwise, which a 16-bit CG stack (FP(P)
+  // rounded to 16 bits) turns into whole steps of its pixels.
+  ColumnShape best;
+  if (maxRowStep * 63. * (1. + 1e-4) + 3. > 48.)
+    return best;
+  double cost = 0.;
+  auto   consider = [&](int w, int q, int e) {
+    if (double(64 * q - 1) * maxRowStep * (1. + 1e-4) + 4. > 64. * e)
+      return;
+    // instructions of a slice per wavefront, times the wavefronts a SIMD gets (at least
+    // four: below that the slices' latency, not the instructions, sets the time)
+    const double waves = double(nu) * np * ((nv + 64 * q - 1) / (64 * q)) / 1024.;
+    const double t = (20. + 2. * e + 8. * q) * std::max(waves, 4.);
+    if (!best.q || t < cost)
+    {
+      best = { w, q, e };
+      cost = t;
+    }
+  };
+#define RTKHIP_CONSIDER(WW, QQ, EE) consider(WW, QQ, EE);
+  RTKHIP_COLUMN_SHAPES(RTKHIP_CONSIDER)
+#undef RTKHIP_CONSIDER
+  return best;
+}
+
 JosephView *
 UploadViews(int np, const double * proj_to_vol, const double * source, hipStream_t s)
 {
@@ -1949,16 +2233,19 @@ rtkhip_joseph_forward_project(const int proj_dim[3], const int vol_dim[3], const
     JosephView * dv = UploadViews(np, proj_to_vol, source, s);
     const size_t nvox = size_t(vol_dim[0]) * vol_dim[1] * vol_dim[2];
     auto &       dT = g_joseph.volT[s];
-    dT.Resize(nvox);
-    dim3 tg((vol_dim[0] + 31) / 32, (vol_dim[2] + 31) / 32, vol_dim[1]);
-    hipLaunchKernelGGL(transpose_xz_kernel, tg, dim3(256), 0, s, dev_vol, dT.get(), vol_dim[0], vol_dim[1],
-                       vol_dim[2]);
-    RTKHIP_CHECK_LAUNCH();
+    auto         copyZFastest = [&] {
+      dT.Resize(nvox);
+      dim3 tg((vol_dim[0] + 31) / 32, (vol_dim[2] + 31) / 32, vol_dim[1]);
+      hipLaunchKernelGGL(transpose_xz_kernel, tg, dim3(256), 0, s, dev_vol, dT.get(), vol_dim[0], vol_dim[1],
+                         vol_dim[2]);
+      RTKHIP_CHECK_LAUNCH();
+    };
     // Ray clip (.hxx:216-218): understood pixel->source, hence inverted.
     const double infClip = 1. - superior_clip, supClip = 1. - inferior_clip;
     dim3         grid((nu + 15) / 16, np, (nv + 15) / 16);
     if (samples)
     {
+      copyZFastest();
       auto & dc = g_joseph.count[s];
       dc.Resize(1);
       RTKHIP_CHECK(hipMemsetAsync(dc.get(), 0, sizeof(unsigned long long), s));
@@ -1973,29 +2260,54 @@ rtkhip_joseph_forward_project(const int proj_dim[3], const int vol_dim[3], const
     }
     else
     {
-      // detector columns vertical in the volume: the gather (same tables as the gather
+      // detector columns vertical in the volume: whole columns (same tables as the gather
       // backprojection, kept across calls with the same geometry)
-      int       freeRows = 1;
-      bool      forward = false;
-      const int nblocks =
-        int(PrepareGather(proj_dim, vol_dim, proj_to_vol, source, inferior_clip, superior_clip, s, freeRows, &forward));
-      if (nblocks >= 0 && forward)
+      int         freeRows = 1;
+      double      maxRowStep = 0.;
+      ColumnShape shape;
+      if (PrepareGather(proj_dim, vol_dim, proj_to_vol, source, inferior_clip, superior_clip, s, freeRows,
+                        &maxRowStep) >= 0)
+        shape = ChooseColumnShape(maxRowStep, nu, nv, np);
+      // heights of a column in the y-fastest copy: a zero below and one above the volume, at
+      // least one run, whole 16-byte chunks.  Flat volumes, whose copy would be far larger
+      // than they are, keep the per-ray kernel.
+      const size_t pitch = std::max<size_t>(64 * size_t(std::max(shape.e, 1)), (size_t(vol_dim[1]) + 5) & ~size_t(3));
+      const size_t padded = pitch * vol_dim[0] * vol_dim[2];
+      if (shape.q && padded < (size_t(1) << 32) && padded <= 4 * nvox + (size_t(1) << 24) && vol_dim[2] <= 65535)
       {
-        dim3 fg((nu + 15) / 16, np, (nv + kFRows - 1) / kFRows);
-        // XCD-contiguous workgroups over the whole grid when the volume and its
-        // transposed copy fit well in the 256 MB last-level cache (256^3 <- 90 x 512^2:
-        // 5.50 -> 4.73 ms; 4.82 ms within bands), within each row band otherwise
-        // (512^3 <- 720 x 1024^2: 318 -> 283 ms; 340 ms over the whole grid)
-        const int xcdOrder = 2 * size_t(vol_dim[0]) * vol_dim[1] * vol_dim[2] * sizeof(float) <= (size_t(192) << 20) ? 1 : 2;
-        hipLaunchKernelGGL(joseph_fp_gather_kernel, fg, dim3(256), 0, s, dv, g_joseph.gviews[s].get(),
-                           g_joseph.gcols[s].get(), g_joseph.gaxis[s].get(), nu, nv, dev_proj_in, dev_proj_out,
-                           dev_vol, dT.get(), vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1],
-                           vol_spacing[2], infClip, supClip, xcdOrder);
+        dT.Resize(padded);
+        dim3 tg((vol_dim[0] + 31) / 32, unsigned((pitch + 31) / 32), vol_dim[2]);
+        hipLaunchKernelGGL(transpose_xy_kernel, tg, dim3(256), 0, s, dev_vol, dT.get(), vol_dim[0], vol_dim[1],
+                           int(pitch));
+        RTKHIP_CHECK_LAUNCH();
+        dim3 fg((nu + shape.w - 1) / shape.w, np, (nv + 64 * shape.q - 1) / (64 * shape.q));
+        // XCD-contiguous workgroups over the whole grid when the copy fits well in the
+        // 256 MB last-level cache, within each row band otherwise
+        const int xcdOrder = padded * sizeof(float) <= (size_t(96) << 20) ? 1 : 2;
+#define RTKHIP_FCOL(WW, QQ, EE)                                                                                      \
+  if (shape.w == WW && shape.q == QQ && shape.e == EE)                                                               \
+    hipLaunchKernelGGL((joseph_fp_column_kernel<WW, QQ, EE>), fg, dim3(64 * WW), 0, s, g_joseph.gviews[s].get(),     \
+                       g_joseph.gcols[s].get(), g_joseph.gaxis[s].get(), nu, nv, dev_proj_in, dev_proj_out,          \
+                       dT.get() + 1, int(pitch), vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1], \
+                       vol_spacing[2], xcdOrder);
+        RTKHIP_COLUMN_SHAPES(RTKHIP_FCOL)
+#undef RTKHIP_FCOL
+        if (const int n = g_joseph.gplanSingle[s])
+        {
+          RTKHIP_CHECK_LAUNCH();
+          hipLaunchKernelGGL(joseph_fp_single_kernel, dim3(unsigned(n), unsigned((nv + 63) / 64)), dim3(64), 0, s, dv,
+                             g_joseph.gsingle[s].get(), nu, nv, dev_proj_in, dev_proj_out, dT.get() + 1, int(pitch),
+                             vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1], vol_spacing[2],
+                             infClip, supClip);
+        }
       }
       else
+      {
+        copyZFastest();
         hipLaunchKernelGGL(joseph_kernel<false>, grid, dim3(256), 0, s, dv, nu, nv, dev_proj_in, dev_proj_out,
                            dev_vol, dT.get(), vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1],
                            vol_spacing[2], infClip, supClip, nullptr);
+      }
       RTKHIP_CHECK_LAUNCH();
     }
   });
