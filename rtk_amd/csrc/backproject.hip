@@ -19,7 +19,8 @@
 //  * Many views per launch: the volume is read and written once per launch,
 //    the per-view matrices are wave-uniform (scalar loads).
 //  * Everything else (X-path views, ITK generic interpolation, non-zero
-//    y-dependence of u or w) runs in a per-voxel general kernel.
+//    y-dependence of u or w) runs in the same kernel's TILT form: the same staging, with
+//    u, v and w of every voxel computed from the whole matrix.
 #include "common.h"
 
 #include <hip/hip_bf16.h>
@@ -109,6 +110,42 @@ FootprintLane(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, fl
   return make_int4(u0, v0, fits ? W : -1, H | (fits && inside ? kInside : 0));
 }
 
+// The same for a matrix whose u and w depend on y too: all eight corners.
+__device__ __forceinline__ int4
+FootprintTilted(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi, int nu, int nv)
+{
+  float umin = FLT_MAX, umax = -FLT_MAX, vmin = FLT_MAX, vmax = -FLT_MAX, smin = 1.f, smax = -1.f;
+#pragma unroll
+  for (int q = 0; q < 8; q++)
+  {
+    const float x = (q & 1) ? xhi : xlo, y = (q & 2) ? yhi : ylo, z = (q & 4) ? zhi : zlo;
+    const float w = c.c[8] + c.c[9] * x + c.c[10] * y + c.c[11] * z;
+    const float rw = __builtin_amdgcn_rcpf(w);
+    const float u = (c.c[0] + c.c[1] * x + c.c[2] * y + c.c[3] * z) * rw;
+    const float v = (c.c[4] + c.c[5] * x + c.c[6] * y + c.c[7] * z) * rw;
+    const float sgn = (w > 0.f) ? 1.f : (w < 0.f ? -1.f : 0.f);
+    umin = fminf(umin, u);
+    umax = fmaxf(umax, u);
+    vmin = fminf(vmin, v);
+    vmax = fmaxf(vmax, v);
+    smin = fminf(smin, sgn);
+    smax = fmaxf(smax, sgn);
+  }
+  if (!(smin == smax && smin != 0.f) || !(umin <= umax) || !(vmin <= vmax) || !(umax - umin < 1e6f) ||
+      !(vmax - vmin < 1e6f))
+    return make_int4(0, 0, -1, 0);
+  // nothing of the view, half a pixel of border included, can reach the block
+  if (umax < -1.f || umin > float(nu) || vmax < -1.f || vmin > float(nv))
+    return make_int4(0, 0, 0, 0);
+  const int  u0 = max(int(floorf(fmaxf(umin, -2.f))) - 1, 0) & ~3, v0 = max(int(floorf(fmaxf(vmin, -2.f))) - 1, 0);
+  const int  u1 = min(int(floorf(fminf(umax, float(nu)))) + 2, nu - 1);
+  const int  v1 = min(int(floorf(fminf(vmax, float(nv)))) + 2, nv - 1);
+  const int  W = u1 - u0 + 1, H = v1 - v0 + 1;
+  const bool inside = umin >= kEdge && umax <= float(nu - 1) - kEdge && vmin >= kEdge && vmax <= float(nv - 1) - kEdge;
+  const bool fits = W > 0 && H > 0 && W <= kTileU && H <= kTileV;
+  return make_int4(u0, v0, fits ? W : -1, H | (fits && inside ? kInside : 0));
+}
+
 // Each thread accumulates a column of NJ voxels along y; a workgroup is 16 (x) x 16
 // (z) columns, a wavefront an 8 x 8 (x, z) patch.  Each view's detector footprint of
 // the workgroup's voxel block is staged in LDS: the footprint of view p + 1 is loaded
@@ -143,8 +180,80 @@ Load4(const TP * p, float * d)
   }
 }
 
-template <typename TP, bool FDK, int NJ, bool VEC>
-__global__ __launch_bounds__(256) void bp_lds_kernel(const ViewCoef * __restrict__ views, int nviews,
+// itk::LinearInterpolateImageFunction (2-D) on the projection, in the
+// transposed frame RTK uses (first index = original v, second = original u).
+template <typename TP>
+__device__ __forceinline__ float
+ItkLinear(const TP * pp, int nu, int nv, float tu, float tv)
+{
+  // tu indexes original v (size nv), tv indexes original u (size nu).
+  const int n0 = nv, n1 = nu;
+  int       b0 = int(floorf(tu)), b1 = int(floorf(tv));
+  b0 = b0 < 0 ? 0 : b0;
+  b1 = b1 < 0 ? 0 : b1;
+  const float d0 = tu - float(b0), d1 = tv - float(b1);
+  auto        at = [&](int a, int b) { return LoadPix(pp, long(a) * nu + b); }; // a: v row, b: u col
+  const float v00 = at(b0, b1);
+  if (d0 <= 0.f && d1 <= 0.f)
+    return v00;
+  if (d1 <= 0.f)
+    return (b0 + 1 > n0 - 1) ? v00 : v00 + (at(b0 + 1, b1) - v00) * d0;
+  if (d0 <= 0.f)
+    return (b1 + 1 > n1 - 1) ? v00 : v00 + (at(b0, b1 + 1) - v00) * d1;
+  if (b0 + 1 > n0 - 1)
+    return (b1 + 1 > n1 - 1) ? v00 : v00 + (at(b0, b1 + 1) - v00) * d1;
+  const float v10 = at(b0 + 1, b1);
+  const float vx0 = v00 + (v10 - v00) * d0;
+  if (b1 + 1 > n1 - 1)
+    return vx0;
+  const float v11 = at(b0 + 1, b1 + 1), v01 = at(b0, b1 + 1);
+  const float vx1 = v01 + (v11 - v01) * d0;
+  return vx0 + (vx1 - vx0) * d1;
+}
+
+// One voxel of one view, read from global memory: per-voxel perspective, per-view border
+// rule.
+template <typename TP, bool FDK>
+__device__ __forceinline__ float
+UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float x, float y, float z)
+{
+  // written out, so that every caller rounds alike: one ulp of u or v can decide whether
+  // a voxel is inside the border
+  auto        row = [&](const float * m) { return fmaf(m[3], z, fmaf(m[2], y, fmaf(m[1], x, m[0]))); };
+  const float rw = 1.f / row(c.c + 8), u = row(c.c) * rw, v = row(c.c + 4) * rw;
+  if (itk)
+  {
+    // Inside iff -0.5 <= idx < n - 0.5 in both directions.
+    if (v >= -0.5f && v < float(nv) - 0.5f && u >= -0.5f && u < float(nu) - 0.5f)
+      return (FDK ? rw * rw : 1.f) * ItkLinear(pp, nu, nv, v, u);
+    return 0.f;
+  }
+  const float uf = floorf(u), vf = floorf(v);
+  if (uf >= 0.f && int(uf) < nu - 1 && vf >= 0.f && int(vf) < nv - 1)
+  {
+    const int   ui = int(uf), vi = int(vf);
+    const float fu = u - uf, fv = v - vf;
+    const long  o = long(vi) * nu + ui;
+    const float a = LoadPix(pp, o), b = LoadPix(pp, o + nu), cc = LoadPix(pp, o + 1), d = LoadPix(pp, o + nu + 1);
+    const float t0 = (1.f - fv) * a + fv * b;
+    const float t1 = (1.f - fv) * cc + fv * d;
+    return (FDK ? rw * rw : 1.f) * ((1.f - fu) * t0 + fu * t1);
+  }
+  return 0.f;
+}
+
+// TILT: the views' u and w may depend on y and their border rule may be ITK's (border[p],
+// null: all optimized).  u, v and w of every voxel come from the whole matrix; a view whose
+// footprint lies inside the detector (one comparison per block) runs with no border test,
+// about 32 instructions an update, others test and clamp every tap; both read the stage.
+// Footprints larger than the stage and optimized views among tilted ones read global memory
+// voxel by voxel.  Same sums as a thread per voxel in global memory, bit for bit.
+// VALU-bound; 203 x 181 x 221 <- 157 x 301 x 257, FP16 stack: 3.24 ms (a thread per voxel,
+// every tap from global memory) -> 1.9 ms (690 G updates/s; 2184 workgroups are 1.7 rounds
+// of the chip, so the last round is two thirds full).
+template <typename TP, bool FDK, int NJ, bool VEC, bool TILT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 1))) void bp_lds_kernel(const ViewCoef * __restrict__ views,
+                                                     const int * __restrict__ border, int nviews,
                                                      const TP * __restrict__ proj, int nu, int nv,
                                                      const float * vol_in, float * vol_out, int nx, int ny, int nz,
                                                      float ci, float cj, float ck)
@@ -152,7 +261,11 @@ __global__ __launch_bounds__(256) void bp_lds_kernel(const ViewCoef * __restrict
   __shared__ __align__(16) float stage[2][kTileV * kTileStride];
   __shared__ int4  rects[2][kPlaceViews]; // footprints (u0, v0, W, H) of two chunks of views
   const int        t = threadIdx.x;
-  const int        bx0 = blockIdx.x * 16, bz0 = blockIdx.y * 16, j0 = blockIdx.z * NJ;
+  // blocks x fastest, then z, then y; TILT numbers them along grid x alone (any volume size)
+  const unsigned   nbx = (nx + 15) / 16, nbz = (nz + 15) / 16;
+  const int        bx0 = (TILT ? blockIdx.x % nbx : blockIdx.x) * 16;
+  const int        bz0 = (TILT ? blockIdx.x / nbx % nbz : blockIdx.y) * 16;
+  const int        j0 = (TILT ? blockIdx.x / (nbx * nbz) : blockIdx.z) * NJ;
   const int        i = bx0 + (t & 7) + 8 * ((t >> 6) & 1);
   const int        k = bz0 + ((t >> 3) & 7) + 8 * (t >> 7);
   const bool       live = i < nx && k < nz;
@@ -238,7 +351,8 @@ __global__ __launch_bounds__(256) void bp_lds_kernel(const ViewCoef * __restrict
   auto      place = [&](int chunk) {
     const int q = chunk * kPlaceViews + (t & 63);
     if (q < nviews)
-      rects[chunk & 1][t & 63] = FootprintLane(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv);
+      rects[chunk & 1][t & 63] = TILT ? FootprintTilted(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv)
+                                      : FootprintLane(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv);
   };
   auto rectOf = [&](int q, int & u0, int & v0, int & W, int & H, bool & in) {
     const int4 r = rects[(q / kPlaceViews) & 1][q % kPlaceViews];
@@ -268,10 +382,92 @@ __global__ __launch_bounds__(256) void bp_lds_kernel(const ViewCoef * __restrict
     }
     if (wave == 0 && p % kPlaceViews == 0 && p + kPlaceViews < nviews)
       place(p / kPlaceViews + 1);
+    if constexpr (TILT)
+    {
+      const ViewCoef & c = views[p];
+      const bool       itk = border && border[p] == RTKHIP_BORDER_ITK_LINEAR;
+      const TP *       pp = proj + long(p) * projStride;
+      if (live && cW > 0 && itk)
+      {
+        const float * S = stage[b];
+        const float   bw = fmaf(c.c[9], x, c.c[8]), bu = fmaf(c.c[1], x, c.c[0]), bv = fmaf(c.c[5], x, c.c[4]);
+        const int     off = -(cv0 * kTileStride + cu0);
+        auto          coords = [&](int jj, float & rw, float & u, float & v) {
+          const float y = y0 + float(jj);
+          // the reciprocal's one Newton step is its correctly rounded value (Markstein 1990:
+          // from an approximation within an ulp), what a division gives
+          const float w = fmaf(c.c[11], z, fmaf(c.c[10], y, bw)), r = __builtin_amdgcn_rcpf(w);
+          rw = fmaf(fmaf(-w, r, 1.f), r, r);
+          u = fmaf(c.c[3], z, fmaf(c.c[2], y, bu)) * rw;
+          v = fmaf(c.c[7], z, fmaf(c.c[6], y, bv)) * rw;
+        };
+        // ITK's rule near the border, and where a coordinate is whole: inside half a pixel
+        // around the detector; along each axis the second tap is read, and weighted, only if
+        // it exists and its weight is not zero (it may hold a NaN)
+        auto bordered = [&](float rw, float u, float v, float & a) {
+          const float fu = u - floorf(u), fv = v - floorf(v);
+          const int   iu = int(floorf(u)), iv = int(floorf(v));
+          const bool  in = v >= -0.5f && v < float(nv) - 0.5f && u >= -0.5f && u < float(nu) - 0.5f;
+          const bool  twoU = iu >= 0 && iu < nu - 1 && fu > 0.f, twoV = iv >= 0 && iv < nv - 1 && fv > 0.f;
+          const int   lc = min(max(iu - cu0, 0), cW - 1), lr = min(max(iv - cv0, 0), cH - 1);
+          const int   lc1 = min(lc + (twoU ? 1 : 0), cW - 1), lr1 = min(lr + (twoV ? 1 : 0), cH - 1);
+          const float *r0 = S + lr * kTileStride, *r1 = S + lr1 * kTileStride;
+          const float v00 = r0[lc], v10 = r1[lc], v01 = r0[lc1], v11 = r1[lc1];
+          const float t0 = twoV ? fmaf(v10 - v00, fv, v00) : v00, t1 = twoV ? fmaf(v11 - v01, fv, v01) : v01;
+          const float val = twoU ? fmaf(t1 - t0, fu, t0) : t0;
+          a = in ? fmaf(FDK ? rw * rw : 1.f, val, a) : a;
+        };
+        if (cIn && jn == NJ)
+        {
+#pragma unroll
+          for (int jj = 0; jj < NJ; jj++)
+          {
+            float rw, u, v;
+            coords(jj, rw, u, v);
+            // inside the detector: truncation is the floor, every tap is staged
+            const float fu = __builtin_amdgcn_fractf(u), fv = __builtin_amdgcn_fractf(v);
+            if (__any(fu * fv == 0.f))
+              bordered(rw, u, v, acc[jj]);
+            else
+            {
+              const float * s0 = S + (int(__umul24(unsigned(int(v)), unsigned(kTileStride))) + (int(u) + off));
+              const float   t0 = fmaf(s0[kTileStride] - s0[0], fv, s0[0]);
+              const float   t1 = fmaf(s0[kTileStride + 1] - s0[1], fv, s0[1]);
+              acc[jj] = fmaf(FDK ? rw * rw : 1.f, fmaf(t1 - t0, fu, t0), acc[jj]);
+            }
+          }
+        }
+        else
+        {
+#pragma unroll
+          for (int jj = 0; jj < NJ; jj++)
+            if (jj < jn)
+            {
+              float rw, u, v;
+              coords(jj, rw, u, v);
+              bordered(rw, u, v, acc[jj]);
+            }
+        }
+      }
+      else if (live && cW != 0)
+      {
+        // the sums rotate through the registers, so that the loop stays one (large) body
+#pragma unroll 1
+        for (int jj = 0; jj < NJ; jj++)
+        {
+          const float first =
+            acc[0] + (jj < jn ? UpdateGeneral<TP, FDK>(c, itk, pp, nu, nv, x, y0 + float(jj), z) : 0.f);
+#pragma unroll
+          for (int q = 0; q + 1 < NJ; q++)
+            acc[q] = acc[q + 1];
+          acc[NJ - 1] = first;
+        }
+      }
+    }
     // per-view limits of the fast path (wave-uniform)
     const bool  viewFast = jn == NJ && cW > 0;
     const float fvLo = float(cv0), fvHi = float(min(nv - 1, cv0 + cH - 1));
-    if (live && cW != 0)
+    if (!TILT && live && cW != 0)
     {
       const ViewCoef & c = views[p];
       const float      w = c.c[8] + c.c[9] * x + c.c[11] * z;
@@ -385,85 +581,6 @@ __global__ __launch_bounds__(256) void bp_lds_kernel(const ViewCoef * __restrict
   }
 }
 
-// itk::LinearInterpolateImageFunction (2-D) on the projection, in the
-// transposed frame RTK uses (first index = original v, second = original u).
-template <typename TP>
-__device__ __forceinline__ float
-ItkLinear(const TP * pp, int nu, int nv, float tu, float tv)
-{
-  // tu indexes original v (size nv), tv indexes original u (size nu).
-  const int n0 = nv, n1 = nu;
-  int       b0 = int(floorf(tu)), b1 = int(floorf(tv));
-  b0 = b0 < 0 ? 0 : b0;
-  b1 = b1 < 0 ? 0 : b1;
-  const float d0 = tu - float(b0), d1 = tv - float(b1);
-  auto        at = [&](int a, int b) { return LoadPix(pp, long(a) * nu + b); }; // a: v row, b: u col
-  const float v00 = at(b0, b1);
-  if (d0 <= 0.f && d1 <= 0.f)
-    return v00;
-  if (d1 <= 0.f)
-    return (b0 + 1 > n0 - 1) ? v00 : v00 + (at(b0 + 1, b1) - v00) * d0;
-  if (d0 <= 0.f)
-    return (b1 + 1 > n1 - 1) ? v00 : v00 + (at(b0, b1 + 1) - v00) * d1;
-  if (b0 + 1 > n0 - 1)
-    return (b1 + 1 > n1 - 1) ? v00 : v00 + (at(b0, b1 + 1) - v00) * d1;
-  const float v10 = at(b0 + 1, b1);
-  const float vx0 = v00 + (v10 - v00) * d0;
-  if (b1 + 1 > n1 - 1)
-    return vx0;
-  const float v11 = at(b0 + 1, b1 + 1), v01 = at(b0, b1 + 1);
-  const float vx1 = v01 + (v11 - v01) * d0;
-  return vx0 + (vx1 - vx0) * d1;
-}
-
-// General kernel: per-voxel perspective, per-view border rule.
-template <typename TP, bool FDK>
-__global__ __launch_bounds__(256) void bp_general_kernel(const ViewCoef * __restrict__ views,
-                                                          const int * __restrict__ border, int nviews,
-                                                          const TP * __restrict__ proj, int nu, int nv,
-                                                          const float * vol_in, float * vol_out, int nx, int ny,
-                                                          int nz, float ci, float cj, float ck)
-{
-  const long idx = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  const long n = long(nx) * ny * nz;
-  if (idx >= n)
-    return;
-  const int   i = int(idx % nx);
-  const int   j = int((idx / nx) % ny);
-  const int   k = int(idx / (long(nx) * ny));
-  const float x = float(i) - ci, y = float(j) - cj, z = float(k) - ck;
-  float       acc = vol_in ? vol_in[idx] : 0.f;
-  const long  projStride = long(nu) * nv;
-  for (int p = 0; p < nviews; p++)
-  {
-    const ViewCoef & c = views[p];
-    const float      w = c.c[8] + c.c[9] * x + c.c[10] * y + c.c[11] * z;
-    const float      rw = 1.f / w;
-    const float      u = (c.c[0] + c.c[1] * x + c.c[2] * y + c.c[3] * z) * rw;
-    const float      v = (c.c[4] + c.c[5] * x + c.c[6] * y + c.c[7] * z) * rw;
-    const TP *       pp = proj + long(p) * projStride;
-    if (border && border[p] == RTKHIP_BORDER_ITK_LINEAR)
-    {
-      // Inside iff -0.5 <= idx < n - 0.5 in both directions.
-      if (v >= -0.5f && v < float(nv) - 0.5f && u >= -0.5f && u < float(nu) - 0.5f)
-        acc += (FDK ? rw * rw : 1.f) * ItkLinear(pp, nu, nv, v, u);
-      continue;
-    }
-    const float uf = floorf(u), vf = floorf(v);
-    if (uf >= 0.f && int(uf) < nu - 1 && vf >= 0.f && int(vf) < nv - 1)
-    {
-      const int   ui = int(uf), vi = int(vf);
-      const float fu = u - uf, fv = v - vf;
-      const long  o = long(vi) * nu + ui;
-      const float a = LoadPix(pp, o), b = LoadPix(pp, o + nu), cc = LoadPix(pp, o + 1), d = LoadPix(pp, o + nu + 1);
-      const float t0 = (1.f - fv) * a + fv * b;
-      const float t1 = (1.f - fv) * cc + fv * d;
-      acc += (FDK ? rw * rw : 1.f) * ((1.f - fu) * t0 + fu * t1);
-    }
-  }
-  vol_out[idx] = acc;
-}
-
 // Per-(thread, stream) cache of the uploaded view coefficients.
 struct CoefCache
 {
@@ -480,26 +597,24 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
        const float * vin, float * vout, int nx, int ny, int nz, float ci, float cj, float ck, hipStream_t s)
 {
   const TP * p = static_cast<const TP *>(proj);
-  if (column)
-  {
-    dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + kNJ - 1) / kNJ);
-    // the vector staging path addresses a view with 32-bit byte offsets
-    const bool vec = (nu & 3) == 0 && (reinterpret_cast<size_t>(p) & 15) == 0 &&
-                     size_t(nu) * size_t(nv) * sizeof(TP) < (size_t(1) << 32);
-    if (vec)
-      hipLaunchKernelGGL((bp_lds_kernel<TP, FDK, kNJ, true>), grid, dim3(256), 0, s, dcoef, nviews, p, nu, nv, vin,
-                         vout, nx, ny, nz, ci, cj, ck);
-    else
-      hipLaunchKernelGGL((bp_lds_kernel<TP, FDK, kNJ, false>), grid, dim3(256), 0, s, dcoef, nviews, p, nu, nv, vin,
-                         vout, nx, ny, nz, ci, cj, ck);
-  }
+  dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + kNJ - 1) / kNJ);
+  if (!column)
+    grid = dim3(grid.x * grid.y * grid.z);
+  // the vector staging path addresses a view with 32-bit byte offsets
+  const bool vec = (nu & 3) == 0 && (reinterpret_cast<size_t>(p) & 15) == 0 &&
+                   size_t(nu) * size_t(nv) * sizeof(TP) < (size_t(1) << 32);
+#define RTKHIP_BP(VV, TT)                                                                                            \
+  hipLaunchKernelGGL((bp_lds_kernel<TP, FDK, kNJ, VV, TT>), grid, dim3(256), 0, s, dcoef, dborder, nviews, p, nu, nv, \
+                     vin, vout, nx, ny, nz, ci, cj, ck)
+  if (column && vec)
+    RTKHIP_BP(true, false);
+  else if (column)
+    RTKHIP_BP(false, false);
+  else if (vec)
+    RTKHIP_BP(true, true);
   else
-  {
-    const long n = long(nx) * ny * nz;
-    dim3       grid(unsigned((n + 255) / 256));
-    hipLaunchKernelGGL((bp_general_kernel<TP, FDK>), grid, dim3(256), 0, s, dcoef, dborder, nviews, p, nu, nv, vin,
-                       vout, nx, ny, nz, ci, cj, ck);
-  }
+    RTKHIP_BP(false, true);
+#undef RTKHIP_BP
   RTKHIP_CHECK_LAUNCH();
 }
 
