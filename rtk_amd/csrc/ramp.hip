@@ -18,6 +18,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -855,46 +856,124 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void ra
 // Hermitian, and IFFT(K FFT(a + i b)) = (h * a) + i (h * b) exactly.
 constexpr int kMaxRadices = 24;
 
+// cos(2 pi m / R) and sin(2 pi m / R) at compile time: Taylor series on [0, pi].
+constexpr double
+SeriesCosSin(int m, int R, bool sine)
+{
+  const double x = 2 * 3.141592653589793238462643383279502884 * m / R;
+  // around pi the series is evaluated from pi, where it converges faster
+  const bool   flip = 4 * m > R && 4 * m < 3 * R;
+  const double y = flip ? x - 3.141592653589793238462643383279502884
+                        : (4 * m >= 3 * R ? x - 2 * 3.141592653589793238462643383279502884 : x);
+  double       term = sine ? y : 1., sum = term;
+  for (int k = sine ? 2 : 1; k < 30; k += 2)
+  {
+    term *= -y * y / (k * (k + 1.));
+    sum += term;
+  }
+  return flip ? -sum : sum;
+}
+template <int R>
+struct Roots
+{
+  float c[R], s[R];
+  constexpr Roots()
+    : c{}
+    , s{}
+  {
+    for (int m = 0; m < R; m++)
+    {
+      c[m] = float(SeriesCosSin(m, R, false));
+      s[m] = float(SeriesCosSin(m, R, true));
+    }
+  }
+};
+
+// R-point DFT in registers.  Odd R: the sums and differences of v[m] and v[R - m] meet real
+// factors only, (R - 1)^2 real FMAs instead of the 4 R^2 of R complex products per output.
+template <int R, bool INV>
+__device__ __forceinline__ void
+DftMixed(float2 (&v)[R])
+{
+  if constexpr (R == 2)
+  {
+    const float2 a = v[0], b = v[1];
+    v[0] = make_float2(a.x + b.x, a.y + b.y);
+    v[1] = make_float2(a.x - b.x, a.y - b.y);
+  }
+  else if constexpr (R == 4)
+    DftReg<4, INV>(v);
+  else
+  {
+    constexpr Roots<R> root;
+    constexpr int      H = (R - 1) / 2;
+    float2             a[H], b[H], first = v[0];
+#pragma unroll
+    for (int m = 0; m < H; m++)
+    {
+      a[m] = make_float2(v[m + 1].x + v[R - 1 - m].x, v[m + 1].y + v[R - 1 - m].y);
+      b[m] = make_float2(v[m + 1].x - v[R - 1 - m].x, v[m + 1].y - v[R - 1 - m].y);
+      first.x += a[m].x;
+      first.y += a[m].y;
+    }
+#pragma unroll
+    for (int q = 1; q <= H; q++)
+    {
+      float2 e = v[0], o = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int m = 0; m < H; m++)
+      {
+        const float c = root.c[((m + 1) * q) % R], s = root.s[((m + 1) * q) % R];
+        e.x = fmaf(c, a[m].x, e.x);
+        e.y = fmaf(c, a[m].y, e.y);
+        o.x = fmaf(s, b[m].x, o.x);
+        o.y = fmaf(s, b[m].y, o.y);
+      }
+      // forward: e - i o at q, e + i o at R - q
+      const float2 lo = make_float2(e.x + o.y, e.y - o.x), hi = make_float2(e.x - o.y, e.y + o.x);
+      v[q] = INV ? hi : lo;
+      v[R - q] = INV ? lo : hi;
+      // v[0] is read again by the next q: outputs q, R - q >= 1 leave it alone, and the
+      // inputs are all in a and b
+    }
+    v[0] = first;
+  }
+}
+
 // One pass of radix R over `batch` transforms of N points stored back to back:
 // butterfly j reads src[j + r N/R], multiplies by W_{NS R}^{r (j mod NS)} (tw[t] =
 // exp(-2 pi i t / N)), applies the R-point DFT and writes dst[(j - j mod NS) R + j mod NS
-// + r NS].
+// + r NS].  The quotients are of numbers far below 2^24: one FP32 product each, with half a
+// unit of margin.
 template <int R, bool INV>
 __device__ __forceinline__ void
 MixedPass(const float2 * __restrict__ src, float2 * __restrict__ dst, const float2 * __restrict__ tw, int N, int NS,
           int batch)
 {
-  const int NR = N / R, step = N / (NS * R);
-  float2    root[R];
-#pragma unroll
-  for (int m = 0; m < R; m++)
-    root[m] = INV ? conj2(tw[m * NR]) : tw[m * NR];
+  const int   NR = N / R, step = N / (NS * R);
+  const float invNR = 1.f / float(NR), invNS = 1.f / float(NS);
   for (int jj = threadIdx.x; jj < batch * NR; jj += blockDim.x)
   {
-    const int      f = jj / NR, j = jj - f * NR, k = j % NS;
+    const int      f = int((float(jj) + 0.5f) * invNR), j = jj - f * NR;
+    const int      k = j - int((float(j) + 0.5f) * invNS) * NS;
     const float2 * sp = src + f * N;
     float2 *       dp = dst + f * N;
     float2         v[R];
 #pragma unroll
     for (int r = 0; r < R; r++)
       v[r] = sp[j + r * NR];
-#pragma unroll
-    for (int r = 1; r < R; r++)
-      v[r] = cmul(v[r], INV ? conj2(tw[r * k * step]) : tw[r * k * step]);
-    const int o = (j - k) * R + k;
-#pragma unroll
-    for (int q = 0; q < R; q++)
-    {
-      float2 acc = v[0];
+    if (NS > 1)
 #pragma unroll
       for (int r = 1; r < R; r++)
       {
-        const float2 t = cmul(v[r], root[(r * q) % R]);
-        acc.x += t.x;
-        acc.y += t.y;
+        const float2 w = tw[r * k * step];
+        v[r] = cmul(v[r], INV ? conj2(w) : w);
       }
-      dp[o + q * NS] = acc;
-    }
+    DftMixed<R, INV>(v);
+    const int o = (j - k) * R + k;
+#pragma unroll
+    for (int q = 0; q < R; q++)
+      dp[o + q * NS] = v[q];
   }
 }
 
@@ -965,46 +1044,59 @@ PaddedSample(const float * row, const WeightView * wv, float dx, float dy, int j
   return 0.f;
 }
 
-// Ramp filter of two detector rows per workgroup (rows 2 blockIdx.x and 2 blockIdx.x + 1
-// of the slab, in (view, row) order) for any padded length N with prime factors <= 13.
-// K: the full N-point kernel spectrum.  LDS: 2N complex values.
-template <typename TO>
-__global__ __launch_bounds__(256) void ramp_mixed_kernel(const float * __restrict__ in, TO * __restrict__ out, int nu,
-                                                          int nv, long nrows, int N, int zeroext,
-                                                          const float2 * __restrict__ tw,
+// Ramp filter of 2F detector rows per workgroup (rows 2F blockIdx.x .. of the slab, in
+// (view, row) order) for any padded length N with prime factors <= 13.  K: the full N-point
+// kernel spectrum.  LDS: 2FN complex values, then (LDSTW) the N twiddles.  F pairs of rows
+// give every thread a butterfly: one pair of 605 points (5 x 11 x 11) has 55 for a pass of
+// radix 11.  Bound by LDS accesses and their latency.  157 x 257 rows of 301, padded to 605,
+// FP16 out: 1.47 ms (one pair a workgroup, R^2 complex products a butterfly) -> 0.21 ms.
+template <typename TO, bool LDSTW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void ramp_mixed_kernel(const float * __restrict__ in, TO * __restrict__ out, int nu,
+                                                          int nv, long nrows, int N, int F, int zeroext,
+                                                          const float2 * __restrict__ tables,
                                                           const float2 * __restrict__ K, const int * __restrict__ rad,
                                                           int nrad, int next, const float * __restrict__ mirror,
                                                           const WeightView * __restrict__ wviews, float dx, float dy)
 {
   extern __shared__ float2 lds[];
-  const long r0 = 2 * long(blockIdx.x);
-  const bool two = r0 + 1 < nrows;
-  const int  p0 = int(r0 / nv), j0 = int(r0 % nv);
-  const int  p1 = two ? int((r0 + 1) / nv) : p0, j1 = two ? int((r0 + 1) % nv) : j0;
-  const float * row0 = in + r0 * nu;
-  const float * row1 = in + (two ? r0 + 1 : r0) * nu;
-  const WeightView * wv0 = wviews ? wviews + p0 : nullptr;
-  const WeightView * wv1 = wviews ? wviews + p1 : nullptr;
-  for (int n = threadIdx.x; n < N; n += blockDim.x)
-    lds[n] = make_float2(PaddedSample(row0, wv0, dx, dy, j0, nu, zeroext, next, mirror, n),
-                         two ? PaddedSample(row1, wv1, dx, dy, j1, nu, zeroext, next, mirror, n) : 0.f);
-  __syncthreads();
-  float2 * z = MixedFFT<false>(lds, lds + N, tw, N, rad, nrad, 1);
-  float2 * other = z == lds ? lds + N : lds;
-  for (int k = threadIdx.x; k < N; k += blockDim.x)
-    z[k] = cmul(z[k], K[k]);
-  __syncthreads();
-  z = MixedFFT<true>(z, other, tw, N, rad, nrad, 1);
-  const float scale = 1.f / float(N);
-  TO *        o0 = out + r0 * nu;
-  TO *        o1 = out + (r0 + 1) * nu;
-  for (int i = threadIdx.x; i < nu; i += blockDim.x)
+  const long     r0 = 2 * F * long(blockIdx.x);
+  const int      rows = int(min(long(2 * F), nrows - r0));
+  const float2 * tw = tables;
+  if constexpr (LDSTW)
   {
-    const float2 v = z[zeroext + i];
-    StoreOut(o0, i, v.x * scale);
-    if (two)
-      StoreOut(o1, i, v.y * scale);
+    float2 * t = lds + 2 * F * N;
+    for (int n = threadIdx.x; n < N; n += blockDim.x)
+      t[n] = tables[n];
+    tw = t;
   }
+  float * ldsf = reinterpret_cast<float *>(lds);
+  // row r0 + 2 f is the real part of transform f, row r0 + 2 f + 1 its imaginary part
+  for (int r = 0; r < 2 * F; r++)
+  {
+    const long         row = r0 + (r < rows ? r : 0);
+    const int          p = int(row / nv), j = int(row - long(p) * nv);
+    const float *      src = in + row * nu;
+    const WeightView * wv = wviews ? wviews + p : nullptr;
+    for (int n = threadIdx.x; n < N; n += blockDim.x)
+      ldsf[2 * ((r >> 1) * N + n) + (r & 1)] =
+        r < rows ? PaddedSample(src, wv, dx, dy, j, nu, zeroext, next, mirror, n) : 0.f;
+  }
+  __syncthreads();
+  float2 * z = MixedFFT<false>(lds, lds + F * N, tw, N, rad, nrad, F);
+  float2 * other = z == lds ? lds + F * N : lds;
+  for (int k = threadIdx.x; k < N; k += blockDim.x)
+  {
+    const float2 h = K[k];
+    for (int f = 0; f < F; f++)
+      z[f * N + k] = cmul(z[f * N + k], h);
+  }
+  __syncthreads();
+  z = MixedFFT<true>(z, other, tw, N, rad, nrad, F);
+  const float   scale = 1.f / float(N);
+  const float * zf = reinterpret_cast<const float *>(z);
+  for (int r = 0; r < rows; r++)
+    for (int i = threadIdx.x; i < nu; i += blockDim.x)
+      StoreOut(out, (r0 + r) * nu + i, zf[2 * ((r >> 1) * N + zeroext + i) + (r & 1)] * scale);
 }
 
 // Filters every detector column (along v) of view blockIdx.y, columns 2F blockIdx.x ..
@@ -1248,20 +1340,36 @@ rtkhip_ramp_filter(const int proj_dim[3], int xpad, const double * kernel, int t
           im = c ? -kernel[2 * h + 1] : kernel[2 * h + 1];
         },
         s);
-      const size_t lds = sizeof(float2) * 2 * size_t(N);
-      RTKHIP_REQUIRE(lds <= MaxLds(), RTKHIP_ERR_UNSUPPORTED, "ramp_filter: padded row does not fit in LDS");
-      const long nrows = long(nv) * np;
+      // pairs of rows per workgroup: a butterfly of the largest radix for most threads, in
+      // at most 40 KB of LDS (four workgroups per CU); the twiddles beside them where they fit
+      const int    maxRadix = *std::max_element(radices.begin(), radices.end());
+      const int    F = int(std::max<size_t>(
+        1, std::min<size_t>((256 * maxRadix + N / 2) / N, (size_t(40) << 10) / (sizeof(float2) * 2 * size_t(N)))));
+      const size_t data = sizeof(float2) * 2 * size_t(F) * N, withTw = data + sizeof(float2) * N;
+      RTKHIP_REQUIRE(data <= MaxLds(), RTKHIP_ERR_UNSUPPORTED, "ramp_filter: padded row does not fit in LDS");
+      const bool   ldsTw = withTw <= size_t(64) << 10 && withTw <= MaxLds();
+      const size_t lds = ldsTw ? withTw : data;
+      const long   nrows = long(nv) * np, groups = (nrows + 2 * F - 1) / (2 * F);
       RTKHIP_REQUIRE((nrows + 1) / 2 <= 2147483647L, RTKHIP_ERR_UNSUPPORTED, "ramp_filter: too many rows");
-      dim3 grid(unsigned((nrows + 1) / 2));
+      dim3 grid{ unsigned(groups) };
+#define RTKHIP_RAMPM2(TO, LT)                                                                                        \
+  hipLaunchKernelGGL((ramp_mixed_kernel<TO, LT>), grid, dim3(256), lds, s, dev_in, static_cast<TO *>(dev_out), nu,  \
+                     nv, nrows, N, F, int(zeroext), t.tw(), t.K(N), t.rad(N), t.nrad, trunc_next, dmirror, dw, dx, dy)
 #define RTKHIP_RAMPM(TO)                                                                                             \
-  hipLaunchKernelGGL(ramp_mixed_kernel<TO>, grid, dim3(256), lds, s, dev_in, static_cast<TO *>(dev_out), nu, nv,    \
-                     nrows, N, int(zeroext), t.tw(), t.K(N), t.rad(N), t.nrad, trunc_next, dmirror, dw, dx, dy)
+  do                                                                                                                 \
+  {                                                                                                                  \
+    if (ldsTw)                                                                                                       \
+      RTKHIP_RAMPM2(TO, true);                                                                                       \
+    else                                                                                                             \
+      RTKHIP_RAMPM2(TO, false);                                                                                      \
+  } while (0)
       if (out_dtype == RTKHIP_F32)
         RTKHIP_RAMPM(float);
       else if (out_dtype == RTKHIP_F16)
         RTKHIP_RAMPM(__half);
       else
         RTKHIP_RAMPM(__hip_bfloat16);
+#undef RTKHIP_RAMPM2
 #undef RTKHIP_RAMPM
       RTKHIP_CHECK_LAUNCH();
       return;
