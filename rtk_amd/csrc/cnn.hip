@@ -12,13 +12,10 @@
 //
 // Kernels (gfx950):
 //  * 32->32 layers (forward and data gradient) are implicit GEMMs on
-//    v_mfma_f32_16x16x32_bf16: M = 16 voxels along x, N = 16 output channels,
-//    K = 32 input channels per tap, 27 taps accumulated in FP32.  A workgroup is
-//    16 (x) x 4 (y) x 4 (z) voxels; wave w owns z-plane w and four M-tiles (y rows).
-//    The block's input with its one-voxel halo is staged in LDS once; A fragments
-//    are 16-byte channel chunks of neighbouring voxels read from there (1 KB per
-//    instruction, conflict-free), B fragments 16-byte chunks of the weights.  Bias, ReLU
-//    and the ReLU-derivative mask of the data gradient are fused into the epilogue.
+//    v_mfma_f32_16x16x32_bf16: M = 16 output channels, N = 16 voxels along x,
+//    K = 32 input channels per tap, 27 taps accumulated in FP32, from an LDS block of the
+//    input with its halo.  Bias, ReLU and the ReLU-derivative mask of the data gradient
+//    are fused into the epilogue.
 //  * The 32->32 weight gradients are GEMMs over the voxels on the same instruction,
 //    their operands transposed by the LDS reads.
 //  * The 1->32 and 32->1 layers and their weight gradients run on the VALU in FP32 (they
@@ -95,95 +92,138 @@ __global__ __launch_bounds__(256) void conv_in_kernel(const float * __restrict__
 // out[v][co] = epilogue(b[co] + sum_t sum_ci W[t][co][ci] in[v + d(t)][ci])
 // epilogue: optional ReLU; optional mask (out *= mask[v][co] > 0).
 // w layout [27][32 co][32 ci] BF16.
-constexpr int kRowsY = 4; // y rows (M-tiles) per wave: a block is 16 x kRowsY x 4 voxels (8: 2.09 ms vs 1.85 ms at 256^3, occupancy)
+//
+// A workgroup is 16 (x) x kRowsY (y) x 4 (z) voxels, a wavefront one z plane.  The block's
+// input with a one-voxel halo is staged in LDS once (zero outside the volume).  A wavefront
+// reads each input row of its three planes once, as three fragments (dx = -1, 0, 1), and
+// multiplies it for the up to three output rows it feeds (dy), against the nine taps of the
+// plane held in registers: 90 LDS fragments for 432 matrix instructions instead of one for
+// every two.  Per output the taps still come in the order (dz, dy, dx), so sums are the same
+// as tap by tap.  Products are W (co) x voxels, so a lane ends with four channels of a voxel
+// and stores 8 bytes.  256^3 layer: 1.87 ms (497 TFLOP/s; a fragment per tap and output row,
+// LDS-bound) -> 1.08 ms (860 TFLOP/s; the matrix units alone need 0.37, the rest is staging,
+// which one other workgroup per CU overlaps).
+constexpr int kRowsY = 8;
 
 template <bool RELU, bool MASK>
-__global__ __launch_bounds__(256) void conv32_mfma_kernel(const bf16_t * __restrict__ in,
+__global__ __launch_bounds__(256, 2) void conv32_mfma_kernel(const bf16_t * __restrict__ in,
                                                            const bf16_t * __restrict__ w,
                                                            const float * __restrict__ bias,
                                                            const bf16_t * __restrict__ mask, bf16_t * __restrict__ out,
                                                            int X, int Y, int Z, int tilesX, int tilesY, int tilesZ)
 {
-  // The block's input with a one-voxel halo, 18 (x) x 6 (y) x 6 (z) voxels of 32
-  // channels, is staged in LDS once (zero outside the volume); every tap's A
-  // fragment is then a conflict-free 1 KB LDS read instead of a global load.
   constexpr int HX = 18, HY = kRowsY + 2, HZ = 6, NCHUNK = HX * HY * HZ * 4;
   __shared__ bf16x8 halo[NCHUNK];
   const int  lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  long       blk = blockIdx.x;
-  const int  tx = int(blk % tilesX);
-  blk /= tilesX;
-  const int  ty = int(blk % tilesY);
-  blk /= tilesY;
-  const int  tz = int(blk % tilesZ);
-  const int  b = int(blk / tilesZ);
+  unsigned   blk = blockIdx.x;
+  const int  tx = int(blk % unsigned(tilesX));
+  blk /= unsigned(tilesX);
+  const int  ty = int(blk % unsigned(tilesY));
+  blk /= unsigned(tilesY);
+  const int  tz = int(blk % unsigned(tilesZ));
+  const int  b = int(blk / unsigned(tilesZ));
   const int  z = tz * 4 + wave;
   const int  y0 = ty * kRowsY;
-  const int  xl = lane & 15;  // voxel of this lane's A row (x offset in the block)
+  const int  xl = lane & 15;  // voxel of this lane's column (x offset in the block)
   const int  kg = lane >> 4;  // channel group: ci = 8 kg .. 8 kg + 7
   const long volBase = long(b) * Z * Y * X;
 
   const bf16x8 zero8 = bf16x8{ bf16_t(0.f), bf16_t(0.f), bf16_t(0.f), bf16_t(0.f),
                                bf16_t(0.f), bf16_t(0.f), bf16_t(0.f), bf16_t(0.f) };
-  for (int c = threadIdx.x; c < NCHUNK; c += 256)
+  // every load of the block is in flight before the first is stored
+  constexpr int PER = (NCHUNK + 255) / 256;
+  bf16x8        reg[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++)
   {
-    const int part = c & 3, vi = c >> 2;
+    const int c = int(threadIdx.x) + 256 * q, vi = c >> 2;
     const int xs = tx * 16 - 1 + vi % HX, ys = y0 - 1 + (vi / HX) % HY, zs = tz * 4 - 1 + vi / (HX * HY);
-    bf16x8    v = zero8;
-    if (xs >= 0 && xs < X && ys >= 0 && ys < Y && zs >= 0 && zs < Z)
-      v = *reinterpret_cast<const bf16x8 *>(in + ((volBase + (long(zs) * Y + ys) * X + xs) * C + 8 * part));
-    halo[c] = v;
+    reg[q] = zero8;
+    if (c < NCHUNK && unsigned(xs) < unsigned(X) && unsigned(ys) < unsigned(Y) && unsigned(zs) < unsigned(Z))
+      reg[q] = *reinterpret_cast<const bf16x8 *>(in + ((volBase + (long(zs) * Y + ys) * X + xs) * C + 8 * (c & 3)));
   }
-  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PER; q++)
+    if (int(threadIdx.x) + 256 * q < NCHUNK)
+      halo[threadIdx.x + 256 * q] = reg[q];
 
   floatx4 acc[kRowsY][2];
 #pragma unroll
   for (int r = 0; r < kRowsY; r++)
     for (int nn = 0; nn < 2; nn++)
       acc[r][nn] = floatx4{ 0.f, 0.f, 0.f, 0.f };
-
-  for (int t = 0; t < T; t++)
+  // the plane's nine taps, both halves of the output channels
+  bf16x8 wt[9][2];
+  auto   taps = [&](int dz) {
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+      for (int nn = 0; nn < 2; nn++)
+        wt[t][nn] = *reinterpret_cast<const bf16x8 *>(w + (long(9 * dz + t) * C + 16 * nn + xl) * C + 8 * kg);
+  };
+  taps(0);
+  __syncthreads();
+#pragma unroll 1
+  for (int dz = 0; dz < 3; dz++)
   {
-    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-    const bf16x8 b0 = *reinterpret_cast<const bf16x8 *>(w + (long(t) * C + (lane & 15)) * C + 8 * kg);
-    const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(w + (long(t) * C + 16 + (lane & 15)) * C + 8 * kg);
-    const int    hbase = ((wave + dz + 1) * HY + dy + 1) * HX + xl + dx + 1;
+    const bf16x8 * plane = halo + ((wave + dz) * HY * HX + xl) * 4 + kg;
+#pragma unroll
+    for (int i = 0; i < HY; i++)
+    {
+      bf16x8 a[3];
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++)
+        a[dx] = plane[(i * HX + dx) * 4];
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++)
+      {
+        const int r = i - dy;
+        if (r < 0 || r >= kRowsY)
+          continue;
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+          for (int nn = 0; nn < 2; nn++)
+            acc[r][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[3 * dy + dx][nn], a[dx], acc[r][nn], 0, 0, 0);
+      }
+    }
+    if (dz < 2)
+      taps(dz + 1);
+  }
+  const int x = tx * 16 + xl;
+  if (z >= Z || x >= X)
+    return;
+  // D layout: lane holds rows (channels) 4 * (lane / 16) + q of column (voxel) lane % 16
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int nn = 0; nn < 2; nn++)
+  {
+    const int co = 16 * nn + 4 * kg;
+    float     bb[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      bb[q] = bias ? bias[co + q] : 0.f;
 #pragma unroll
     for (int r = 0; r < kRowsY; r++)
     {
-      const bf16x8 a = halo[(hbase + r * HX) * 4 + kg];
-      acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0, acc[r][0], 0, 0, 0);
-      acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b1, acc[r][1], 0, 0, 0);
-    }
-  }
-  if (z >= Z)
-    return;
-  // D layout: lane holds rows (voxels) 4*(lane/16)+q, column (channel) lane%16.
-#pragma unroll
-  for (int r = 0; r < kRowsY; r++)
-  {
-    const int y = y0 + r;
-    if (y >= Y)
-      continue;
-#pragma unroll
-    for (int nn = 0; nn < 2; nn++)
-    {
-      const int   co = 16 * nn + (lane & 15);
-      const float bb = bias ? bias[co] : 0.f;
+      const int y = y0 + r;
+      if (y >= Y)
+        continue;
+      const long o = (volBase + (long(z) * Y + y) * X + x) * C + co;
+      bf16x4     m, res;
+      if (MASK)
+        m = *reinterpret_cast<const bf16x4 *>(mask + o);
 #pragma unroll
       for (int q = 0; q < 4; q++)
       {
-        const int x = tx * 16 + 4 * (lane >> 4) + q;
-        if (x >= X)
-          continue;
-        const long o = (volBase + (long(z) * Y + y) * X + x) * C + co;
-        float      v = acc[r][nn][q] + bb;
+        float v = acc[r][nn][q] + bb[q];
         if (RELU)
           v = fmaxf(v, 0.f);
         if (MASK)
-          v = (float(mask[o]) > 0.f) ? v : 0.f;
-        out[o] = bf16_t(v);
+          v = (float(m[q]) > 0.f) ? v : 0.f;
+        res[q] = bf16_t(v);
       }
+      *reinterpret_cast<bf16x4 *>(out + o) = res;
     }
   }
 }
@@ -508,26 +548,30 @@ __global__ __launch_bounds__(256) void wgrad_io_kernel(const float * __restrict_
   }
 }
 
-// dst(slot) = sum over the workgroups' slices, in a fixed order: a workgroup takes 64
-// slots, four quarters of the slices, in four chains each.  `where` maps a slot to its
-// place and factor.
+// dst(slot) = sum over the workgroups' slices, in a fixed order: a workgroup takes 16
+// slots (64-byte reads), its 16 rows of threads every 16th slice each.  `where` maps a slot
+// to its place and factor.
 template <class F>
 __device__ __forceinline__ void
 WgReduce(const float * __restrict__ part, int nslots, int nslices, F && where)
 {
-  __shared__ float red[4][64];
-  const int slot = blockIdx.x * 64 + (threadIdx.x & 63), quarter = threadIdx.x >> 6;
-  float     v[4] = { 0.f, 0.f, 0.f, 0.f };
+  __shared__ float red[16][17];
+  const int slot = blockIdx.x * 16 + (threadIdx.x & 15), row = threadIdx.x >> 4;
+  float     v = 0.f;
   if (slot < nslots)
-    for (int b = quarter; b < nslices; b += 16)
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (b + 4 * q < nslices)
-          v[q] += part[size_t(b + 4 * q) * nslots + slot];
-  red[quarter][threadIdx.x & 63] = (v[0] + v[1]) + (v[2] + v[3]);
+#pragma unroll 8
+    for (int b = row; b < nslices; b += 16)
+      v += part[size_t(b) * nslots + slot];
+  red[row][threadIdx.x & 15] = v;
   __syncthreads();
-  if (quarter == 0 && slot < nslots)
-    where(slot, (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]));
+  if (row == 0 && slot < nslots)
+  {
+    float s = red[0][threadIdx.x];
+#pragma unroll
+    for (int r = 1; r < 16; r++)
+      s += red[r][threadIdx.x];
+    where(slot, s);
+  }
 }
 
 // 32 -> 32 layer: W and b lie together, in the order of the slots.
@@ -778,8 +822,10 @@ rtkhip_cnn_backward(rtkhip_cnn * net, const float * dev_out, const float * dev_t
                        net->partial.get());
     RTKHIP_CHECK_LAUNCH();
     const unsigned g = unsigned((n + 255) / 256);
-    const int  tilesX = (X + 15) / 16, tilesY = (Y + kRowsY - 1) / kRowsY, tilesZ = (Z + 3) / 4;
-    const long nb = long(B) * tilesX * tilesY * tilesZ;
+    const int  tilesX = (X + 15) / 16, tilesY = (Y + 3) / 4, tilesZ = (Z + 3) / 4; // of the weight gradients
+    const int  convY = (Y + kRowsY - 1) / kRowsY;                                  // of the data gradients
+    const long nb = long(B) * tilesX * tilesY * tilesZ, nconv = long(B) * tilesX * convY * tilesZ;
+    RTKHIP_REQUIRE(nb < (1L << 31), RTKHIP_ERR_UNSUPPORTED, "cnn: volume too large");
     const int  ng = int(std::min<long>(nb, kWgGroups));
     net->wpart.Resize(size_t(ng) * kWgSums);
     float * part = net->wpart.get();
@@ -787,7 +833,7 @@ rtkhip_cnn_backward(rtkhip_cnn * net, const float * dev_out, const float * dev_t
       hipLaunchKernelGGL(wgrad_io_kernel, dim3(ng), dim3(256), 0, s, f, m, part, X, Y, Z, tilesX, tilesY, tilesZ,
                          int(nb));
       RTKHIP_CHECK_LAUNCH();
-      hipLaunchKernelGGL(wgrad_io_reduce_kernel, dim3((kWgIoSums + 63) / 64), dim3(256), 0, s, part, ng, g, factor,
+      hipLaunchKernelGGL(wgrad_io_reduce_kernel, dim3((kWgIoSums + 15) / 16), dim3(256), 0, s, part, ng, g, factor,
                          last);
       RTKHIP_CHECK_LAUNCH();
     };
@@ -805,11 +851,11 @@ rtkhip_cnn_backward(rtkhip_cnn * net, const float * dev_out, const float * dev_t
       hipLaunchKernelGGL(wgrad32_mfma_kernel, dim3(ng), dim3(256), 0, s, aprev, cur, part, X, Y, Z, tilesX, tilesY,
                          tilesZ, int(nb));
       RTKHIP_CHECK_LAUNCH();
-      hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((kWgSums + 63) / 64), dim3(256), 0, s, part, ng,
+      hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((kWgSums + 15) / 16), dim3(256), 0, s, part, ng,
                          G + kMidBase + l * kMidSize);
       RTKHIP_CHECK_LAUNCH();
-      hipLaunchKernelGGL((conv32_mfma_kernel<false, true>), dim3(unsigned(nb)), dim3(256), 0, s, cur,
-                         net->wb.get() + size_t(l) * T * C * C, nullptr, aprev, nxt, X, Y, Z, tilesX, tilesY,
+      hipLaunchKernelGGL((conv32_mfma_kernel<false, true>), dim3(unsigned(nconv)), dim3(256), 0, s, cur,
+                         net->wb.get() + size_t(l) * T * C * C, nullptr, aprev, nxt, X, Y, Z, tilesX, convY,
                          tilesZ);
       RTKHIP_CHECK_LAUNCH();
       std::swap(cur, nxt);

@@ -48,3 +48,9 @@ def test_gradients_are_exact_on_integers(hip, shape):
     assert loss == pytest.approx(lr, rel=1e-12)
     assert np.any(gr != 0.)
     assert np.array_equal(net.grads(), gr)
+
+
+# the 16 x 8 x 4 tile of the 32 -> 32 layers: one row under, at and over it, and over twice
+@pytest.mark.parametrize("shape", [(2, 4, 7, 15), (1, 5, 8, 16), (1, 3, 9, 18), (1, 4, 17, 32)])
+def test_layers_are_exact_on_integers(hip, shape):
+    test_gradients_are_exact_on_integers(hip, shape)
