@@ -54,3 +54,28 @@ def test_gradients_are_exact_on_integers(hip, shape):
 @pytest.mark.parametrize("shape", [(2, 4, 7, 15), (1, 5, 8, 16), (1, 3, 9, 18), (1, 4, 17, 32)])
 def test_layers_are_exact_on_integers(hip, shape):
     test_gradients_are_exact_on_integers(hip, shape)
+
+
+# layer 6 from three BF16 terms per weight: one voxel, partial and several 16 x 16 columns, several
+# z runs of a workgroup; a5 is exact (layers 2 - 5 pass their input on), so y's error is that of an
+# FP32 sum: at most n 2^-24 of the sum of magnitudes, n < 3 * 864 + 40
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 9, 15, 16), (1, 5, 17, 18), (1, 13, 33, 31)])
+def test_last_layer_to_float_rounding(hip, shape):
+    from oracle import cnn_ref
+    from rtk_amd.warmstart import WarmStartCNN
+    C, T = cnn_ref.C, cnn_ref.T
+    rng = np.random.default_rng(sum(shape))
+    d = {"w1": np.zeros((T, C)), "b1": np.zeros(C), "b6": np.array([0.25])}
+    d["w1"][T // 2] = rng.choice([1., -1., 0.5, -0.25], C)
+    for l in range(2, 6):
+        d[f"w{l}"], d[f"b{l}"] = np.zeros((T, C, C)), np.zeros(C)
+        d[f"w{l}"][T // 2] = np.eye(C)
+    d["w6"] = (rng.standard_normal((T, C)) * 10. ** rng.uniform(-3, 1, (T, C))).astype(np.float32).astype(float)
+    x = torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).bfloat16().float()
+    p = cnn_ref.pack(d)
+    y = WarmStartCNN(params=p, scale=1.).forward(x.cuda()).cpu().numpy()
+    yr, _ = cnn_ref.forward(p, x.numpy().astype(np.float64), 1.)
+    mags = dict(d, w6=np.abs(d["w6"]))
+    bound = 2600 * 2. ** -24 * (cnn_ref.forward(cnn_ref.pack(mags), x.numpy().astype(np.float64), 1.)[0]
+                                + 2 * np.abs(x.numpy()))
+    assert np.all(np.abs(y - yr) <= bound)
