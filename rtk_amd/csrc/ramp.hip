@@ -856,132 +856,70 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void ra
 // Hermitian, and IFFT(K FFT(a + i b)) = (h * a) + i (h * b) exactly.
 constexpr int kMaxRadices = 24;
 
-// cos(2 pi m / R) and sin(2 pi m / R) at compile time: Taylor series on [0, pi].
-constexpr double
-SeriesCosSin(int m, int R, bool sine)
+// d w (INV: d conj(w)), the product with w's imaginary part rounded first: the rounding does
+// not depend on the place it is compiled in, so a filtered 16-bit sample does not either.
+template <bool INV>
+__device__ __forceinline__ float2
+MixedMul(float2 d, float2 w)
 {
-  const double x = 2 * 3.141592653589793238462643383279502884 * m / R;
-  // around pi the series is evaluated from pi, where it converges faster
-  const bool   flip = 4 * m > R && 4 * m < 3 * R;
-  const double y = flip ? x - 3.141592653589793238462643383279502884
-                        : (4 * m >= 3 * R ? x - 2 * 3.141592653589793238462643383279502884 : x);
-  double       term = sine ? y : 1., sum = term;
-  for (int k = sine ? 2 : 1; k < 30; k += 2)
-  {
-    term *= -y * y / (k * (k + 1.));
-    sum += term;
-  }
-  return flip ? -sum : sum;
+  const float px = d.y * w.y, py = d.x * w.y;
+  return INV ? make_float2(fmaf(d.x, w.x, px), fmaf(d.y, w.x, -py)) : make_float2(fmaf(d.x, w.x, -px), fmaf(d.y, w.x, py));
 }
-template <int R>
-struct Roots
-{
-  float c[R], s[R];
-  constexpr Roots()
-    : c{}
-    , s{}
-  {
-    for (int m = 0; m < R; m++)
-    {
-      c[m] = float(SeriesCosSin(m, R, false));
-      s[m] = float(SeriesCosSin(m, R, true));
-    }
-  }
-};
 
-// R-point DFT in registers.  Odd R: the sums and differences of v[m] and v[R - m] meet real
-// factors only, (R - 1)^2 real FMAs instead of the 4 R^2 of R complex products per output.
-template <int R, bool INV>
-__device__ __forceinline__ void
-DftMixed(float2 (&v)[R])
-{
-  if constexpr (R == 2)
-  {
-    const float2 a = v[0], b = v[1];
-    v[0] = make_float2(a.x + b.x, a.y + b.y);
-    v[1] = make_float2(a.x - b.x, a.y - b.y);
-  }
-  else if constexpr (R == 4)
-    DftReg<4, INV>(v);
-  else
-  {
-    constexpr Roots<R> root;
-    constexpr int      H = (R - 1) / 2;
-    float2             a[H], b[H], first = v[0];
-#pragma unroll
-    for (int m = 0; m < H; m++)
-    {
-      a[m] = make_float2(v[m + 1].x + v[R - 1 - m].x, v[m + 1].y + v[R - 1 - m].y);
-      b[m] = make_float2(v[m + 1].x - v[R - 1 - m].x, v[m + 1].y - v[R - 1 - m].y);
-      first.x += a[m].x;
-      first.y += a[m].y;
-    }
-#pragma unroll
-    for (int q = 1; q <= H; q++)
-    {
-      float2 e = v[0], o = make_float2(0.f, 0.f);
-#pragma unroll
-      for (int m = 0; m < H; m++)
-      {
-        const float c = root.c[((m + 1) * q) % R], s = root.s[((m + 1) * q) % R];
-        e.x = fmaf(c, a[m].x, e.x);
-        e.y = fmaf(c, a[m].y, e.y);
-        o.x = fmaf(s, b[m].x, o.x);
-        o.y = fmaf(s, b[m].y, o.y);
-      }
-      // forward: e - i o at q, e + i o at R - q
-      const float2 lo = make_float2(e.x + o.y, e.y - o.x), hi = make_float2(e.x - o.y, e.y + o.x);
-      v[q] = INV ? hi : lo;
-      v[R - q] = INV ? lo : hi;
-      // v[0] is read again by the next q: outputs q, R - q >= 1 leave it alone, and the
-      // inputs are all in a and b
-    }
-    v[0] = first;
-  }
-}
+extern __shared__ float2 mixedLds[];
 
 // One pass of radix R over `batch` transforms of N points stored back to back:
 // butterfly j reads src[j + r N/R], multiplies by W_{NS R}^{r (j mod NS)} (tw[t] =
 // exp(-2 pi i t / N)), applies the R-point DFT and writes dst[(j - j mod NS) R + j mod NS
-// + r NS].  The quotients are of numbers far below 2^24: one FP32 product each, with half a
-// unit of margin.
-template <int R, bool INV>
+// + r NS].  src, dst and (LDSTW) tw are offsets into LDS, so their accesses are LDS
+// instructions and not generic ones.  The quotients are of numbers far below 2^24: one FP32
+// product each, with half a unit of margin.
+template <int R, bool INV, bool LDSTW>
 __device__ __forceinline__ void
-MixedPass(const float2 * __restrict__ src, float2 * __restrict__ dst, const float2 * __restrict__ tw, int N, int NS,
-          int batch)
+MixedPass(int src, int dst, const float2 * __restrict__ tw, int ldsTw, int N, int NS, int batch)
 {
+  auto        W = [&](int t) { return LDSTW ? mixedLds[ldsTw + t] : tw[t]; };
   const int   NR = N / R, step = N / (NS * R);
   const float invNR = 1.f / float(NR), invNS = 1.f / float(NS);
+  float2      root[R];
+#pragma unroll
+  for (int m = 0; m < R; m++)
+    root[m] = W(m * NR);
   for (int jj = threadIdx.x; jj < batch * NR; jj += blockDim.x)
   {
     const int      f = int((float(jj) + 0.5f) * invNR), j = jj - f * NR;
     const int      k = j - int((float(j) + 0.5f) * invNS) * NS;
-    const float2 * sp = src + f * N;
-    float2 *       dp = dst + f * N;
+    const float2 * sp = mixedLds + src + f * N + j;
     float2         v[R];
 #pragma unroll
     for (int r = 0; r < R; r++)
-      v[r] = sp[j + r * NR];
+      v[r] = sp[r * NR];
     if (NS > 1)
 #pragma unroll
       for (int r = 1; r < R; r++)
-      {
-        const float2 w = tw[r * k * step];
-        v[r] = cmul(v[r], INV ? conj2(w) : w);
-      }
-    DftMixed<R, INV>(v);
-    const int o = (j - k) * R + k;
+        v[r] = MixedMul<INV>(v[r], W(r * k * step));
+    float2 * dp = mixedLds + dst + f * N + (j - k) * R + k;
 #pragma unroll
     for (int q = 0; q < R; q++)
-      dp[o + q * NS] = v[q];
+    {
+      float2 acc = v[0];
+#pragma unroll
+      for (int r = 1; r < R; r++)
+      {
+        const float2 t = MixedMul<INV>(v[r], root[(r * q) % R]);
+        acc.x += t.x;
+        acc.y += t.y;
+      }
+      dp[q * NS] = acc;
+    }
   }
 }
 
-// `batch` N-point FFTs of a (b is the other buffer); returns the buffer holding the
+// `batch` N-point FFTs at LDS offset a (b is the other buffer); returns the offset of the
 // result.  The caller synchronises before (input written) and after (result read).
-template <bool INV>
-__device__ float2 *
-MixedFFT(float2 * a, float2 * b, const float2 * __restrict__ tw, int N, const int * __restrict__ rad, int nrad,
+template <bool INV, bool LDSTW>
+__device__ __forceinline__ int
+MixedFFT(int a, int b, const float2 * __restrict__ tw, int ldsTw, int N, const int * __restrict__ rad, int nrad,
          int batch)
 {
   int NS = 1;
@@ -991,29 +929,29 @@ MixedFFT(float2 * a, float2 * b, const float2 * __restrict__ tw, int N, const in
     switch (R)
     {
       case 2:
-        MixedPass<2, INV>(a, b, tw, N, NS, batch);
+        MixedPass<2, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       case 3:
-        MixedPass<3, INV>(a, b, tw, N, NS, batch);
+        MixedPass<3, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       case 4:
-        MixedPass<4, INV>(a, b, tw, N, NS, batch);
+        MixedPass<4, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       case 5:
-        MixedPass<5, INV>(a, b, tw, N, NS, batch);
+        MixedPass<5, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       case 7:
-        MixedPass<7, INV>(a, b, tw, N, NS, batch);
+        MixedPass<7, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       case 11:
-        MixedPass<11, INV>(a, b, tw, N, NS, batch);
+        MixedPass<11, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
       default:
-        MixedPass<13, INV>(a, b, tw, N, NS, batch);
+        MixedPass<13, INV, LDSTW>(a, b, tw, ldsTw, N, NS, batch);
         break;
     }
     __syncthreads();
-    float2 * t = a;
+    const int t = a;
     a = b;
     b = t;
     NS *= R;
@@ -1048,8 +986,11 @@ PaddedSample(const float * row, const WeightView * wv, float dx, float dy, int j
 // (view, row) order) for any padded length N with prime factors <= 13.  K: the full N-point
 // kernel spectrum.  LDS: 2FN complex values, then (LDSTW) the N twiddles.  F pairs of rows
 // give every thread a butterfly: one pair of 605 points (5 x 11 x 11) has 55 for a pass of
-// radix 11.  Bound by LDS accesses and their latency.  157 x 257 rows of 301, padded to 605,
-// FP16 out: 1.47 ms (one pair a workgroup, R^2 complex products a butterfly) -> 0.21 ms.
+// radix 11.  Bound by LDS accesses, their latency and the R^2 complex products of a
+// butterfly (a DFT from sums and differences has a quarter of the products and took the same
+// time, but rounds differently, which a 16-bit stack passes on as whole steps).  157 x 257
+// rows of 301, padded to 605, FP16 out: 1.47 ms (one pair a workgroup, generic loads) ->
+// 0.20 ms.
 template <typename TO, bool LDSTW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void ramp_mixed_kernel(const float * __restrict__ in, TO * __restrict__ out, int nu,
                                                           int nv, long nrows, int N, int F, int zeroext,
@@ -1058,18 +999,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
                                                           int nrad, int next, const float * __restrict__ mirror,
                                                           const WeightView * __restrict__ wviews, float dx, float dy)
 {
-  extern __shared__ float2 lds[];
   const long     r0 = 2 * F * long(blockIdx.x);
   const int      rows = int(min(long(2 * F), nrows - r0));
-  const float2 * tw = tables;
+  const int      ldsTw = 2 * F * N;
   if constexpr (LDSTW)
-  {
-    float2 * t = lds + 2 * F * N;
     for (int n = threadIdx.x; n < N; n += blockDim.x)
-      t[n] = tables[n];
-    tw = t;
-  }
-  float * ldsf = reinterpret_cast<float *>(lds);
+      mixedLds[ldsTw + n] = tables[n];
+  float * ldsf = reinterpret_cast<float *>(mixedLds);
   // row r0 + 2 f is the real part of transform f, row r0 + 2 f + 1 its imaginary part
   for (int r = 0; r < 2 * F; r++)
   {
@@ -1082,18 +1018,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         r < rows ? PaddedSample(src, wv, dx, dy, j, nu, zeroext, next, mirror, n) : 0.f;
   }
   __syncthreads();
-  float2 * z = MixedFFT<false>(lds, lds + F * N, tw, N, rad, nrad, F);
-  float2 * other = z == lds ? lds + F * N : lds;
+  int z = MixedFFT<false, LDSTW>(0, F * N, tables, ldsTw, N, rad, nrad, F);
   for (int k = threadIdx.x; k < N; k += blockDim.x)
   {
     const float2 h = K[k];
     for (int f = 0; f < F; f++)
-      z[f * N + k] = cmul(z[f * N + k], h);
+      mixedLds[z + f * N + k] = MixedMul<false>(mixedLds[z + f * N + k], h);
   }
   __syncthreads();
-  z = MixedFFT<true>(z, other, tw, N, rad, nrad, F);
+  z = MixedFFT<true, LDSTW>(z, F * N - z, tables, ldsTw, N, rad, nrad, F);
   const float   scale = 1.f / float(N);
-  const float * zf = reinterpret_cast<const float *>(z);
+  const float * zf = reinterpret_cast<const float *>(mixedLds + z);
   for (int r = 0; r < rows; r++)
     for (int i = threadIdx.x; i < nu; i += blockDim.x)
       StoreOut(out, (r0 + r) * nu + i, zf[2 * ((r >> 1) * N + zeroext + i) + (r & 1)] * scale);
@@ -1111,11 +1046,10 @@ __global__ __launch_bounds__(256) void column_filter_kernel(const float * in, TO
                                                              const float2 * __restrict__ K,
                                                              const int * __restrict__ rad, int nrad)
 {
-  extern __shared__ float2 lds[];
   const int     p = blockIdx.y, u0 = 2 * F * blockIdx.x, C = 2 * F;
   const float * vin = in + long(p) * nv * nu;
   TO *          vout = out + long(p) * nv * nu;
-  float *       ldsf = reinterpret_cast<float *>(lds);
+  float *       ldsf = reinterpret_cast<float *>(mixedLds);
   for (int e = threadIdx.x; e < N * C; e += blockDim.x)
   {
     const int v = e / C, c = e - v * C, u = u0 + c;
@@ -1123,14 +1057,13 @@ __global__ __launch_bounds__(256) void column_filter_kernel(const float * in, TO
     ldsf[2 * ((c >> 1) * N + v) + (c & 1)] = (v < nv && u < nu) ? vin[long(v) * nu + u] : 0.f;
   }
   __syncthreads();
-  float2 * z = MixedFFT<false>(lds, lds + F * N, tw, N, rad, nrad, F);
-  float2 * other = z == lds ? lds + F * N : lds;
+  int z = MixedFFT<false, false>(0, F * N, tw, 0, N, rad, nrad, F);
   for (int e = threadIdx.x; e < F * N; e += blockDim.x)
-    z[e] = cmul(z[e], K[e % N]);
+    mixedLds[z + e] = MixedMul<false>(mixedLds[z + e], K[e % N]);
   __syncthreads();
-  z = MixedFFT<true>(z, other, tw, N, rad, nrad, F);
+  z = MixedFFT<true, false>(z, F * N - z, tw, 0, N, rad, nrad, F);
   const float   scale = 1.f / float(N);
-  const float * zf = reinterpret_cast<const float *>(z);
+  const float * zf = reinterpret_cast<const float *>(mixedLds + z);
   for (int e = threadIdx.x; e < nv * C; e += blockDim.x)
   {
     const int v = e / C, c = e - v * C, u = u0 + c;
