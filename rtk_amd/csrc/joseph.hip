@@ -340,6 +340,14 @@ struct Walker
   }
 };
 
+// Slices whose taps a ray loads together.  Rays in the middle of their walk for a whole batch
+// (all but the ends of each) have 8 loads in flight, no test per slice and, where their first
+// and last samples show that they stay inside the slice, no index clamp: 19 VALU
+// instructions a sample instead of 38.  251 x 203 x 247 -> 61 tilted views of 389 x 331:
+// 2.41 -> 1.61 ms, now bound by L1 (16 accesses per 8-byte load of a wavefront); batches of 2
+// and 8, 4-byte loads and wavefronts of 8 x 8 rays took 1.62 to 1.73.
+constexpr int kLockBatch = 4;
+
 template <bool COUNT>
 __global__ __launch_bounds__(256) void joseph_kernel(const JosephView * __restrict__ views, int nu, int nv,
                                                       const float * pin, float * pout,
@@ -400,6 +408,8 @@ __global__ __launch_bounds__(256) void joseph_kernel(const JosephView * __restri
     klo = min(klo, __shfl_xor(klo, o, 64));
     khi = max(khi, __shfl_xor(khi, o, 64));
   }
+  klo = __builtin_amdgcn_readfirstlane(klo);
+  khi = __builtin_amdgcn_readfirstlane(khi);
   if (klo <= khi)
   {
     const int     axis = best >> 1, dirSign = (best & 1) ? -1 : 1;
@@ -410,27 +420,68 @@ __global__ __launch_bounds__(256) void joseph_kernel(const JosephView * __restri
     const int     t0 = lock ? (R.ns - kfirst) * dirSign : INT_MAX;
     const int     tEnd = lock ? t0 + R.nmid + 1 : INT_MIN; // R.nmid = -1 when fs == ns
     Walker        wk;
-    for (int s = 0; s < nsl; ++s)
+    // a ray whose first and last middle samples lie inside the slice needs no index clamp;
+    // byte offsets within a slice fit 32 bits (below 2^31 voxels in at least two slices; a
+    // slice along y spans the volume)
+    bool free = false;
+    if (lock && R.nmid > 0 && (axis != 1 || long(nx) * ny * nz < (1L << 30)))
     {
-      if (s >= t0 && s <= tEnd)
+      wk.Init(R.cx + R.stepx, R.cy + R.stepy);
+      const long long X1 = wk.X + (R.nmid - 1) * R.sx32, Y1 = wk.Y + (R.nmid - 1) * R.sy32;
+      free = wk.X >= 0 && X1 >= 0 && int(wk.X >> 32) <= R.nxm2 && int(X1 >> 32) <= R.nxm2 && wk.Y >= 0 && Y1 >= 0 &&
+             int(wk.Y >> 32) <= R.nym2 && int(Y1 >> 32) <= R.nym2;
+    }
+    const unsigned oy = unsigned(axis == 0 ? nz : (axis == 1 ? nx * ny : nx)); // R.oy of the locked rays
+    const long step = dirSign * absOz;
+    for (int s = 0; s < nsl; s += kLockBatch)
+    {
+      const float * slice = buf + __builtin_amdgcn_readfirstlane(kfirst + s * dirSign) * absOz;
+      if (free && s > t0 && s + kLockBatch - 1 < tEnd)
       {
-        const float * bb = buf + (kfirst + s * dirSign) * absOz;
-        const int     t = s - t0;
-        if (t == 0)
+        float lx[kLockBatch], ly[kLockBatch], tap[kLockBatch][4];
+#pragma unroll
+        for (int q = 0; q < kLockBatch; q++)
         {
-          if (R.fs == R.ns)
-            sum += border(R.wOne, bb, R.cx, R.cy);
-          else
-          {
-            sum += border(R.wB, bb, R.cx, R.cy);
-            wk.Init(R.cx + R.stepx, R.cy + R.stepy);
-          }
+          const char *   bb = reinterpret_cast<const char *>(slice + q * step);
+          const unsigned off = 4u * (unsigned(wk.X >> 32) + __umul24(unsigned(wk.Y >> 32), oy));
+          lx[q] = float(unsigned(wk.X)) * 0x1p-32f;
+          ly[q] = float(unsigned(wk.Y)) * 0x1p-32f;
+          wk.X += R.sx32;
+          wk.Y += R.sy32;
+          const float * lo = reinterpret_cast<const float *>(bb + off);
+          const float * hi = reinterpret_cast<const float *>(bb + 4 * size_t(oy) + off);
+          tap[q][0] = lo[0];
+          tap[q][1] = lo[1];
+          tap[q][2] = hi[0];
+          tap[q][3] = hi[1];
         }
-        else if (t <= R.nmid)
-          sum += middle(wk, bb);
-        else
-          sum += border(R.wE, bb, wk.PosX(), wk.PosY());
+#pragma unroll
+        for (int q = 0; q < kLockBatch; q++)
+        {
+          const float lxc = 1.f - lx[q], lyc = 1.f - ly[q];
+          sum += (lxc * lyc) * tap[q][0] + (lx[q] * lyc) * tap[q][1] + (lxc * ly[q]) * tap[q][2] + (lx[q] * ly[q]) * tap[q][3];
+        }
       }
+      else if (s + kLockBatch > t0 && s <= tEnd)
+        for (int sq = max(s, t0); sq <= min(s + kLockBatch - 1, tEnd); sq++)
+        {
+          const float * bb = buf + (kfirst + sq * dirSign) * absOz;
+          const int     t = sq - t0;
+          if (t == 0)
+          {
+            if (R.fs == R.ns)
+              sum += border(R.wOne, bb, R.cx, R.cy);
+            else
+            {
+              sum += border(R.wB, bb, R.cx, R.cy);
+              wk.Init(R.cx + R.stepx, R.cy + R.stepy);
+            }
+          }
+          else if (t <= R.nmid)
+            sum += middle(wk, bb);
+          else
+            sum += border(R.wE, bb, wk.PosX(), wk.PosY());
+        }
     }
   }
   if (hit && !lock)
