@@ -8,7 +8,7 @@
 // Design (CDNA4):
 //  * Circular geometries make the detector column u and the perspective w
 //    independent of the volume y index (RTK's "OptimizedBackprojectionY" case).
-//    Each thread owns a column of NJ voxels along y at fixed (x, z) and keeps
+//    Each thread owns a column of NJ voxels (16, in small volumes 8) along y at fixed (x, z) and keeps
 //    them in registers for the whole launch; per view it computes u, w and the
 //    row step once (one reciprocal) and then only steps v along the column.
 //  * A workgroup is 16 (x) x 16 (z) such columns.  Per view it stages the detector
@@ -51,8 +51,13 @@ struct alignas(16) ViewCoef
 // wave's 8 x 8 voxel patch, whose detector columns span about 16 and whose rows differ
 // by one or two, over distinct LDS banks; it is a multiple of 4, so a lane stages its
 // four pixels with one 16-byte store.
-constexpr int kTileU = 64, kTileV = 48, kTileStride = 76; // staged detector footprint, pixels
-constexpr int kStagePasses = (kTileV + 15) / 16;           // 16 rows per staging pass
+constexpr int kTileU = 64, kTileStride = 76; // staged detector footprint, pixels
+// rows of the footprint of a block of NJ heights; staged 16 rows per pass
+constexpr int
+TileRows(int NJ)
+{
+  return NJ == 8 ? 32 : 48;
+}
 constexpr int kPlaceViews = 64;                            // footprints placed per chunk, one per lane
 // A footprint whose every tap lies at least kEdge pixels inside the detector's
 // interpolation range (0 <= u, v and u < nu - 1, v < nv - 1) is flagged in the bit
@@ -73,9 +78,12 @@ constexpr int   kInside = 1 << 16;
 // (skip the view); W < 0: too large, or w changes sign (read global memory for this
 // view).  One lane evaluates the four (x, z) corners in turn, so a wavefront places
 // the footprints of 64 views at once.
+template <int NJ>
 __device__ __forceinline__ int4
-FootprintLane(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi, int nu, int nv)
+FootprintLane(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi, int nu, int nv,
+              float ylo16, float yhi16)
 {
+  float vin = FLT_MAX, vax = -FLT_MAX; // v over the 16 heights that decide kInside
   float umin = FLT_MAX, umax = -FLT_MAX, vmin = FLT_MAX, vmax = -FLT_MAX, smin = 1.f, smax = -1.f;
 #pragma unroll
   for (int q = 0; q < 4; q++)
@@ -86,6 +94,13 @@ FootprintLane(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, fl
     const float u = (c.c[0] + c.c[1] * x + c.c[3] * z) * rw;
     const float vl = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * ylo) * rw;
     const float vh = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * yhi) * rw;
+    if constexpr (NJ != 16)
+    {
+      const float vl16 = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * ylo16) * rw;
+      const float vh16 = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * yhi16) * rw;
+      vin = fminf(vin, fminf(vl16, vh16));
+      vax = fmaxf(vax, fmaxf(vl16, vh16));
+    }
     const float sgn = (w > 0.f) ? 1.f : (w < 0.f ? -1.f : 0.f);
     umin = fminf(umin, u);
     umax = fmaxf(umax, u);
@@ -105,14 +120,20 @@ FootprintLane(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, fl
   const int  v0 = max(int(fvLo) - 1, 0);
   const int  u1 = min(int(fuHi) + 2, nu - 1), v1 = min(int(fvHi) + 2, nv - 1);
   const int  W = u1 - u0 + 1, H = v1 - v0 + 1;
-  const bool fits = W <= kTileU && H <= kTileV;
-  const bool inside = umin >= kEdge && umax <= float(nu - 1) - kEdge && vmin >= kEdge && vmax <= float(nv - 1) - kEdge;
+  if constexpr (NJ == 16)
+  {
+    vin = vmin;
+    vax = vmax;
+  }
+  const bool fits = W <= kTileU && H <= TileRows(NJ);
+  const bool inside = umin >= kEdge && umax <= float(nu - 1) - kEdge && vin >= kEdge && vax <= float(nv - 1) - kEdge;
   return make_int4(u0, v0, fits ? W : -1, H | (fits && inside ? kInside : 0));
 }
 
 // The same for a matrix whose u and w depend on y too: all eight corners.
 __device__ __forceinline__ int4
-FootprintTilted(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi, int nu, int nv)
+FootprintTilted(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi, int nu, int nv,
+                int rows)
 {
   float umin = FLT_MAX, umax = -FLT_MAX, vmin = FLT_MAX, vmax = -FLT_MAX, smin = 1.f, smax = -1.f;
 #pragma unroll
@@ -142,7 +163,7 @@ FootprintTilted(const ViewCoef & c, float xlo, float xhi, float ylo, float yhi, 
   const int  v1 = min(int(floorf(fminf(vmax, float(nv)))) + 2, nv - 1);
   const int  W = u1 - u0 + 1, H = v1 - v0 + 1;
   const bool inside = umin >= kEdge && umax <= float(nu - 1) - kEdge && vmin >= kEdge && vmax <= float(nv - 1) - kEdge;
-  const bool fits = W > 0 && H > 0 && W <= kTileU && H <= kTileV;
+  const bool fits = W > 0 && H > 0 && W <= kTileU && H <= rows;
   return make_int4(u0, v0, fits ? W : -1, H | (fits && inside ? kInside : 0));
 }
 
@@ -249,8 +270,7 @@ UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float
 // Footprints larger than the stage and optimized views among tilted ones read global memory
 // voxel by voxel.  Same sums as a thread per voxel in global memory, bit for bit.
 // VALU-bound; 203 x 181 x 221 <- 157 x 301 x 257, FP16 stack: 3.24 ms (a thread per voxel,
-// every tap from global memory) -> 1.8 ms (720 G updates/s; 2184 workgroups are 1.7 rounds
-// of the chip, so the last round is two thirds full).
+// every tap from global memory) -> 1.7 ms (750 G updates/s).
 template <typename TP, bool FDK, int NJ, bool VEC, bool TILT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 1))) void bp_lds_kernel(const ViewCoef * __restrict__ views,
                                                      const int * __restrict__ border, int nviews,
@@ -258,6 +278,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
                                                      const float * vol_in, float * vol_out, int nx, int ny, int nz,
                                                      float ci, float cj, float ck)
 {
+  static_assert(NJ == 8 || NJ == 16, "a block is 16 heights or half of them");
+  constexpr int kTileV = TileRows(NJ), kStagePasses = kTileV / 16;
   __shared__ __align__(16) float stage[2][kTileV * kTileStride];
   __shared__ int4  rects[2][kPlaceViews]; // footprints (u0, v0, W, H) of two chunks of views
   const int        t = threadIdx.x;
@@ -280,7 +302,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
   for (int jj = 0; jj < NJ; jj++)
     acc[jj] = 0.f;
 
-  const float x = float(i) - ci, z = float(k) - ck, y0 = float(j0) - cj;
+  // positions along y, and the choice between the tested and the untested column loop (they
+  // round differently), are those of blocks of 16 heights for either NJ, so NJ does not show
+  // in the result; jr: this block's first height among the 16
+  const int   jr = NJ == 16 ? 0 : j0 & 15;
+  const float x = float(i) - ci, z = float(k) - ck, y0 = float(j0) - cj, y16 = float(j0 - jr) - cj;
+  const bool  full16 = NJ == 16 ? jn == NJ : j0 - jr + 16 <= ny;
   const float xlo = float(bx0) - ci, xhi = float(min(bx0 + 15, nx - 1)) - ci;
   const float zlo = float(bz0) - ck, zhi = float(min(bz0 + 15, nz - 1)) - ck;
   const float ylo = y0, yhi = float(j0 + jn - 1) - cj;
@@ -351,8 +378,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
   auto      place = [&](int chunk) {
     const int q = chunk * kPlaceViews + (t & 63);
     if (q < nviews)
-      rects[chunk & 1][t & 63] = TILT ? FootprintTilted(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv)
-                                      : FootprintLane(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv);
+      rects[chunk & 1][t & 63] = TILT ? FootprintTilted(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv, kTileV)
+                                      : FootprintLane<NJ>(views[q], xlo, xhi, ylo, yhi, zlo, zhi, nu, nv, y16,
+                                                          float(min(j0 - jr + 15, ny - 1)) - cj);
   };
   auto rectOf = [&](int q, int & u0, int & v0, int & W, int & H, bool & in) {
     const int4 r = rects[(q / kPlaceViews) & 1][q % kPlaceViews];
@@ -465,7 +493,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
       }
     }
     // per-view limits of the fast path (wave-uniform)
-    const bool  viewFast = jn == NJ && cW > 0;
+    const bool  viewFast = full16 && cW > 0;
     const float fvLo = float(cv0), fvHi = float(min(nv - 1, cv0 + cH - 1));
     if (!TILT && live && cW != 0)
     {
@@ -473,7 +501,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
       const float      w = c.c[8] + c.c[9] * x + c.c[11] * z;
       const float      rw = __builtin_amdgcn_rcpf(w); // 1 ulp
       const float      u = (c.c[0] + c.c[1] * x + c.c[3] * z) * rw;
-      const float      vb = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * y0) * rw;
+      const float      vb = (c.c[4] + c.c[5] * x + c.c[7] * z + c.c[6] * y16) * rw;
       const float      dv = c.c[6] * rw;
       const float      wgt = FDK ? rw * rw : 1.f;
       // The column's detector column pair and whether it runs from the staged
@@ -492,12 +520,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
         // v is monotonic along the column (one FMA per voxel), so its two ends bound
         // every tap: when both pass the border rule and lie in the staged rectangle,
         // the whole column runs without per-voxel tests
-        const float vlast = vb + float(NJ - 1) * dv;
+        const float vlast = vb + float(15) * dv;
         const float vmn = vb < vlast ? vb : vlast, vmx = vb < vlast ? vlast : vb;
         // one combined test (no short-circuit branches): the column lies inside the
         // staged rows [cv0, cv0 + cH - 1) and inside [0, nv - 1), and its detector
         // column pair inside the staged columns; cv0 >= 0 by construction
-        fast = inU & viewFast & (unsigned(lc) < unsigned(cW - 1)) & (floorf(vmn) >= fvLo) & (floorf(vmx) < fvHi);
+        fast = inU & viewFast & (unsigned(lc) < unsigned(cW - 1));
+        if (NJ == 16)
+          fast = fast & (floorf(vmn) >= fvLo) & (floorf(vmx) < fvHi);
+        else
+        {
+          // the 16 heights against the detector, this half against the staged rows
+          const float va = vb + float(jr) * dv, vz = vb + float(jr + NJ - 1) * dv;
+          fast = fast & (floorf(vmn) >= 0.f) & (floorf(vmx) < float(nv - 1)) & (floorf(fminf(va, vz)) >= fvLo) &
+                 (floorf(fmaxf(va, vz)) < fvHi);
+        }
       }
       else
       {
@@ -515,7 +552,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
 #pragma unroll
         for (int jj = 0; jj < NJ; jj++)
         {
-          const float   vv = vb + float(jj) * dv;
+          const float   vv = vb + float(jj + jr) * dv;
           // vv >= 0 on this path: truncation is the floor, and fract(vv) = vv - floor(vv)
           const float   fv = __builtin_amdgcn_fractf(vv);
           // 24-bit multiply: the LDS offset is small and the 32 x 32 form is slower
@@ -532,7 +569,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
 #pragma unroll
         for (int jj = 0; jj < NJ; jj++)
         {
-          const float vv = vb + float(jj) * dv;
+          const float vv = vb + float(jj + jr) * dv;
           const float vf = floorf(vv);
           const int   vi = int(vf);
           if (vf >= 0.f && vi < nv - 1)
@@ -589,7 +626,12 @@ struct CoefCache
 };
 thread_local CoefCache g_cache;
 
-constexpr int kNJ = 16;
+// Heights per block: 16, or 8 where 16 would give fewer workgroups than two rounds of the chip
+// (5 a CU).  A block of 8 stages and sets up as much per view for half the updates, but
+// small volumes leave the chip waiting: 128^3 <- 180 x 256^2 has 512 workgroups of 16.
+// 16 against 8: FDK of 128^3 <- 180 x 256^2 0.49 / 0.40 ms, of 203 x 181 x 221 (tilted, 2184
+// workgroups) 2.10 / 1.96, BP of 256^3 (4096) 2.58 either way, FDK of 512^3 40.0 / 42.8.
+constexpr long kSmallGrid = 2560;
 
 template <typename TP, bool FDK>
 void
@@ -597,15 +639,20 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
        const float * vin, float * vout, int nx, int ny, int nz, float ci, float cj, float ck, hipStream_t s)
 {
   const TP * p = static_cast<const TP *>(proj);
-  dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + kNJ - 1) / kNJ);
+  const long columns = long((nx + 15) / 16) * ((nz + 15) / 16);
+  const int  NJ = columns * ((ny + 15) / 16) < kSmallGrid ? 8 : 16;
+  dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + NJ - 1) / NJ);
   if (!column)
     grid = dim3(grid.x * grid.y * grid.z);
   // the vector staging path addresses a view with 32-bit byte offsets
   const bool vec = (nu & 3) == 0 && (reinterpret_cast<size_t>(p) & 15) == 0 &&
                    size_t(nu) * size_t(nv) * sizeof(TP) < (size_t(1) << 32);
+  auto       launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, dcoef, dborder, nviews, p, nu, nv, vin, vout, nx, ny, nz, ci, cj,
+                       ck);
+  };
 #define RTKHIP_BP(VV, TT)                                                                                            \
-  hipLaunchKernelGGL((bp_lds_kernel<TP, FDK, kNJ, VV, TT>), grid, dim3(256), 0, s, dcoef, dborder, nviews, p, nu, nv, \
-                     vin, vout, nx, ny, nz, ci, cj, ck)
+  NJ == 8 ? launch(bp_lds_kernel<TP, FDK, 8, VV, TT>) : launch(bp_lds_kernel<TP, FDK, 16, VV, TT>)
   if (column && vec)
     RTKHIP_BP(true, false);
   else if (column)
