@@ -235,11 +235,11 @@ __global__ __launch_bounds__(256, 2) void conv32_mfma_kernel(const bf16_t * __re
 // weights enter as three BF16 terms whose sum is the weight exactly (24 bits in three times
 // 8), so every product is exact and the sums are FP32; with fewer sequential additions y's
 // error against 64 bits is a quarter of the tap-by-tap loop's (1.2e-7 of the range, 4.8e-7
-// before).  (An infinite activation gives NaN: a weight's lower terms may be 0.)  A workgroup is a 16 x 16
-// (x, y) column marching along z: per plane its wavefronts write P of the 18 x 18 halo to
-// LDS, then each thread adds 9 values to each of the three outputs the plane feeds, which it
-// keeps in registers; the next plane's activations are loaded meanwhile.  Every activation
-// is read 1.3 times instead of 27.
+// before).  (An infinite activation gives NaN: a weight's lower terms may be 0.)  A workgroup
+// is a 16 x 16 (x, y) column marching along z: per plane its wavefronts write P of the
+// 18 x 18 halo to LDS, then each thread adds 9 values to each of the three outputs the plane
+// feeds, which it keeps in registers; the next plane's activations are loaded meanwhile.
+// Every activation is read 1.3 times instead of 27.
 // 256^3: 1.65 ms (864 VALU FMAs and 108 cached 16-byte loads a voxel) -> 0.27 ms.
 constexpr int kOutX = 16, kOutHX = kOutX + 2, kOutVox = kOutHX * kOutHX; // halo plane
 constexpr int kOutGroups = (kOutVox + 15) / 16;
