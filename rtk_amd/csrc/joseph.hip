@@ -937,9 +937,9 @@ struct GatherColumn
 };
 
 // Per-ray data of the gather: value * |stepMM| (0 for rays the gather must not take);
-// the same value beside the first/last slice (16 bits each) and their weights.
-// Views [p0, p0 + gridDim.y) of the call; gval/gend/gw and colAxis are indexed by the
-// view's position in the chunk.
+// the same value beside the first/last slice (16 bits each) and their weights, both with a
+// detector column's rows contiguous.  Views [p0, p0 + gridDim.y) of the call; gval/gend/gw
+// and colAxis are indexed by the view's position in the chunk.
 template <typename TP>
 __global__ __launch_bounds__(256) void joseph_gather_prep_kernel(
   const JosephView * __restrict__ views, int p0, const signed char * __restrict__ colAxis, int nu, int nv,
@@ -950,14 +950,12 @@ __global__ __launch_bounds__(256) void joseph_gather_prep_kernel(
   const int iu = blockIdx.x * 16 + (threadIdx.x & 15);
   const int jv = blockIdx.z * 16 + (threadIdx.x >> 4);
   const int pl = blockIdx.y, p = p0 + pl;
-  if (iu >= nu || jv >= nv)
-    return;
-  const size_t pix = (size_t(pl) * nv + jv) * nu + iu;
-  const float  value = LoadPix(proj, (long(p) * nv + jv) * nu + iu);
-  Ray          R;
-  float        vn = 0.f;
-  unsigned     e = 0u;
-  float2       w = make_float2(0.f, 0.f);
+  const bool  live = iu < nu && jv < nv;
+  const float value = live ? LoadPix(proj, (long(p) * nv + jv) * nu + iu) : 0.f;
+  Ray         R;
+  float       vn = 0.f;
+  unsigned    e = 0u;
+  float2      w = make_float2(0.f, 0.f);
   if (value != 0.f && SetupRay<true>(views[p], iu, jv, p, nx, ny, nz, spx, spy, spz, infClip, supClip, R))
   {
     if (R.axis == int(colAxis[size_t(pl) * nu + iu]) && isfinite(value))
@@ -969,9 +967,23 @@ __global__ __launch_bounds__(256) void joseph_gather_prep_kernel(
     else
       SplatRay(R, value, acc, accT);
   }
-  gval[pix] = vn;
-  gend[pix] = make_uint2(__float_as_uint(vn), e); // the value again, so the shell reads one 8-byte word
-  gw[pix] = w;
+  if (live)
+    gval[(size_t(pl) * nv + jv) * nu + iu] = vn;
+  // the end slices (with the value again, so that the shell reads one 8-byte word) and their
+  // weights by columns, whose rows the lanes of a shell wavefront are
+  __shared__ uint2  se[16][17];
+  __shared__ float2 sw[16][17];
+  const int a = threadIdx.x & 15, b = threadIdx.x >> 4;
+  se[a][b] = make_uint2(__float_as_uint(vn), e);
+  sw[a][b] = w;
+  __syncthreads();
+  const int cu = blockIdx.x * 16 + b, cv = blockIdx.z * 16 + a;
+  if (cu < nu && cv < nv)
+  {
+    const size_t pix = (size_t(pl) * nu + cu) * nv + cv;
+    gend[pix] = se[b][a];
+    gw[pix] = sw[b][a];
+  }
 }
 
 // Rectangle of rays [u0, u0 + W) x [v0, v0 + H) that can reach the voxel block
@@ -1209,7 +1221,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
                 float       s = 0.f;
                 auto        weight = [&](int r) {
                   const float w = 1.f - fabsf(r == 0 ? y0 : fmaf(bf, float(r), y0));
-                  return r < G ? w : fmaxf(0.f, w);
+                  return r < G ? w : __builtin_amdgcn_fmed3f(w, 0.f, 1.f); // folds into the subtraction
                 };
                 if constexpr (STAGED)
                 {
@@ -1266,7 +1278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
                   const int jv = jref + d0 + r;
                   if (jv < 0 || jv >= nv)
                     continue;
-                  const size_t pix = size_t(p) * viewRays + size_t(jv) * nu + iu;
+                  const size_t pix = (size_t(p) * nu + iu) * nv + jv;
                   const uint2  ve = gend[pix];
                   const float  val = __uint_as_float(ve.x);
                   const int    ns = int(ve.y & 0xffffu), fs = int(ve.y >> 16);
@@ -1317,30 +1329,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
   }
 }
 
-// The voxels of the two outer layers along x and along z, one thread per voxel (voxel
-// indices from `shell`), reading the rays from global memory: these voxels also
-// receive first and last steps, so each candidate (ray, slice) takes its step weight
-// from the ray's first/last slices and, on those, its position clamped into the box.
+// The voxels of the two outer layers along x and along z: a wavefront is 64 heights of one of
+// their columns (indices k nx + i from `shell`), reading the rays from global memory.  These
+// voxels also receive first and last steps, so each candidate (ray, slice) takes its step
+// weight from the ray's first/last slices and, on those, its position clamped into the box.
+// The candidate columns are the same for all 64 heights (scalar loop and table reads), and
+// a column's rows are contiguous in gend and gw.
+// Bound by those reads and by VALU issue together.  512^3 <- 45 of 180 x 1024^2 rays: 4.2 ms
+// (a lane per voxel along the face, its own columns, rows a detector row apart) -> 2.1 ms;
+// 256^3 <- 90 x 512^2: 1.51 -> 0.79 ms.
 __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
   const GatherView * __restrict__ gviews, const GatherColumn * __restrict__ gcols,
-  const signed char * __restrict__ colAxis, int nviews, int nu, int nv, const float * __restrict__ gval,
-  const uint2 * __restrict__ gend, const float2 * __restrict__ gw, const int * __restrict__ shell, int nshell,
-  float * vol, int nx, int ny, int nz)
+  const signed char * __restrict__ colAxis, int nviews, int nu, int nv, const uint2 * __restrict__ gend,
+  const float2 * __restrict__ gw, const int * __restrict__ shell, int ncolumns, float * vol, int nx, int ny, int nz)
 {
   // Workgroups are dealt to the 8 XCDs in turn; XCD x takes a contiguous run of the
-  // shell list instead of every 8th workgroup, so the voxels one XCD's L2 serves lie
+  // columns instead of every 8th workgroup, so the voxels one XCD's L2 serves lie
   // together and read overlapping rays
   const unsigned nb = gridDim.x, full = nb / 8, rem = nb % 8, x = blockIdx.x % 8, q = blockIdx.x / 8;
   const unsigned lb = x * full + min(x, rem) + q;
-  const int      n = int(lb * blockDim.x + threadIdx.x);
-  if (n >= nshell)
+  const unsigned bands = (ny + 63) / 64, w = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w >= unsigned(ncolumns) * bands)
     return;
-  const int    idx = shell[n];
-  const int    i = idx % nx, j = (idx / nx) % ny, k = idx / (nx * ny);
+  const int    column = __builtin_amdgcn_readfirstlane(shell[w / bands]);
+  const int    i = column % nx, j = int(w % bands) * 64 + int(threadIdx.x & 63), k = column / nx;
   const float  cx = 0.5f * float(nx - 1), cy = 0.5f * float(ny - 1), cz = 0.5f * float(nz - 1);
   const float  xc = float(i) - cx, zc = float(k) - cz, yv = float(j) - cy;
   const double xd = double(xc), zd = double(zc);
-  const size_t viewRays = size_t(nu) * nv;
   float        acc = 0.f;
   for (int p = 0; p < nviews; p++)
   {
@@ -1358,8 +1373,8 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
       const float  xb = axis == 0 ? kc : hc + 1.f, zb = axis == 0 ? hc + 1.f : kc;
       const float  ua = (V.pu[3] + V.pu[0] * xa + V.pu[2] * za) * __builtin_amdgcn_rcpf(V.pw[3] + V.pw[0] * xa + V.pw[2] * za);
       const float  ub = (V.pu[3] + V.pu[0] * xb + V.pu[2] * zb) * __builtin_amdgcn_rcpf(V.pw[3] + V.pw[0] * xb + V.pw[2] * zb);
-      const int    iuLo = max(int(ceilf(fminf(ua, ub) - 1e-3f)), 0);
-      const int    iuHi = min(int(floorf(fmaxf(ua, ub) + 1e-3f)), nu - 1);
+      const int    iuLo = __builtin_amdgcn_readfirstlane(max(int(ceilf(fminf(ua, ub) - 1e-3f)), 0));
+      const int    iuHi = __builtin_amdgcn_readfirstlane(min(int(floorf(fmaxf(ua, ub) + 1e-3f)), nu - 1));
       for (int iu = iuLo; iu <= iuHi; iu++)
       {
         // both loads issued before the test, so they overlap
@@ -1381,11 +1396,11 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
         // the rows' slices and values, all loads issued together (rows outside the
         // detector read a clamped row and take weight zero; a ray the gather does not
         // take has value zero and weights zero)
-        const size_t colBase = size_t(p) * viewRays + iu;
+        const size_t colBase = (size_t(p) * nu + iu) * nv;
         uint2        ve[kGRows];
 #pragma unroll
         for (int r = 0; r < kGRows; r++)
-          ve[r] = gend[colBase + size_t(min(max(jref + d0 + r, 0), nv - 1)) * nu];
+          ve[r] = gend[colBase + unsigned(min(max(jref + d0 + r, 0), nv - 1))];
 #pragma unroll
         for (int r = 0; r < kGRows; r++)
         {
@@ -1401,7 +1416,7 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
           float w = wm;
           if (kidx == ns || kidx == fs)
           {
-            const float2 w2 = gw[colBase + size_t(jv) * nu];
+            const float2 w2 = gw[colBase + unsigned(jv)];
             w = (kidx == ns ? w2.x : w2.y) * we;
           }
           acc = fmaf(w, val, acc);
@@ -1409,7 +1424,8 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
       }
     }
   }
-  vol[idx] += acc;
+  if (j < ny)
+    vol[(size_t(k) * ny + j) * nx + i] += acc;
 }
 
 // Forward projection of whole detector columns, for the geometries whose detector
@@ -1885,7 +1901,7 @@ struct JosephCache
   std::map<hipStream_t, DeviceBuffer<float>>        gval;
   std::map<hipStream_t, DeviceBuffer<uint2>>        gend;
   std::map<hipStream_t, DeviceBuffer<float2>>       gw;
-  std::map<hipStream_t, DeviceBuffer<int>>          gshell; // voxels of the outer layers along x and z
+  std::map<hipStream_t, DeviceBuffer<int>>          gshell; // columns of the outer layers along x and z
   std::map<hipStream_t, std::array<int, 3>>         gshellDims;
   std::map<hipStream_t, int>                        gshellCount;
   // the arguments the uploaded tables were made from: a call with the same ones (every
@@ -2120,23 +2136,19 @@ GatherBackproject(long long nblocks, int freeRows, const JosephView * dv, const 
   auto &    gc = g_joseph.gcols[s];
   auto &    ga = g_joseph.gaxis[s];
   auto &    gb = g_joseph.gblocks[s];
-  // the voxels of the two outer layers along x and z, listed once per volume size
+  // the columns of the two outer layers along x and z, listed once per volume size
   auto &                   gs = g_joseph.gshell[s];
   const std::array<int, 3> dims = { nx, ny, nz };
   if (!gs.get() || g_joseph.gshellDims[s] != dims)
   {
-    // consecutive threads take neighbouring voxels of one row across the face (x on the
-    // faces z = 0, 1, nz - 2, nz - 1; z on the faces x = 0, 1, nx - 2, nx - 1), whose
-    // candidate rays lie in the same detector rows
+    // neighbouring columns of a face follow each other: their candidate rays overlap
     std::vector<int> shell;
     for (int z : { 0, 1, nz - 2, nz - 1 })
-      for (int y = 0; y < ny; y++)
-        for (int x = 0; x < nx; x++)
-          shell.push_back((z * ny + y) * nx + x);
+      for (int x = 0; x < nx; x++)
+        shell.push_back(z * nx + x);
     for (int x : { 0, 1, nx - 2, nx - 1 })
-      for (int y = 0; y < ny; y++)
-        for (int z = 2; z < nz - 2; z++)
-          shell.push_back((z * ny + y) * nx + x);
+      for (int z = 2; z < nz - 2; z++)
+        shell.push_back(z * nx + x);
     gs.Resize(shell.size());
     RTKHIP_CHECK(hipMemcpy(gs.get(), shell.data(), sizeof(int) * shell.size(), hipMemcpyHostToDevice));
     g_joseph.gshellDims[s] = dims;
@@ -2171,9 +2183,10 @@ GatherBackproject(long long nblocks, int freeRows, const JosephView * dv, const 
                        dim3(256), 0, s, gv.get() + p0, gc.get() + size_t(p0) * nu, ga.get() + size_t(p0) * nu, c, nu,
                        nv, dval.get(), dend.get(), dw.get(), gb.get(), vol, nx, ny, nz);
     RTKHIP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(joseph_gather_shell_kernel, dim3(unsigned((nshell + 255) / 256)), dim3(256), 0, s,
-                       gv.get() + p0, gc.get() + size_t(p0) * nu, ga.get() + size_t(p0) * nu, c, nu, nv, dval.get(),
-                       dend.get(), dw.get(), gs.get(), nshell, vol, nx, ny, nz);
+    const long shellWaves = long(nshell) * ((ny + 63) / 64);
+    hipLaunchKernelGGL(joseph_gather_shell_kernel, dim3(unsigned((shellWaves + 3) / 4)), dim3(256), 0, s,
+                       gv.get() + p0, gc.get() + size_t(p0) * nu, ga.get() + size_t(p0) * nu, c, nu, nv, dend.get(),
+                       dw.get(), gs.get(), nshell, vol, nx, ny, nz);
     RTKHIP_CHECK_LAUNCH();
   }
 }
