@@ -918,7 +918,10 @@ __global__ __launch_bounds__(256) void joseph_bp_tile_kernel(const JosephView * 
 // of steep cones, ties decided differently in FP64) and rays carrying non-finite values
 // are splatted by the per-ray path instead, so the result is RTK's for every ray.
 
-constexpr int kGTileU = 64, kGTileV = 64, kGStride = 65; // staged ray values: columns x rows
+// Staged ray values: columns x rows.  The row stride spreads a wavefront's rows over the LDS
+// banks and leaves four workgroups a CU; 512^3 <- 180 x 1024^2, all kernels: 79.9 ms with 65,
+// 79.4 with 66, 79.3 with 67 (83.9 with 71: three workgroups).
+constexpr int kGTileU = 64, kGTileV = 64, kGStride = 67;
 constexpr int kGRows = 5;                                // candidate rows per voxel and column
 constexpr int kGNJ = 16;                                 // voxels per thread along y
 
@@ -1061,7 +1064,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
   const int               t = threadIdx.x;
   const int               blk = blocks[blockIdx.x]; // packed (bx, bz, by)
   const int               bx0 = (blk & 0x3ff) * 16, bz0 = ((blk >> 10) & 0x3ff) * 16, j0 = (blk >> 20) * kGNJ;
-  const int               i = bx0 + (t & 15), k = bz0 + (t >> 4);
+  // a wavefront is 8 x 8 columns: their candidate columns differ less than those of 16 x 4
+  // (80.9 ms), for slices along x and along z alike
+  const int               i = bx0 + (t & 7) + 8 * ((t >> 6) & 1), k = bz0 + ((t >> 3) & 7) + 8 * (t >> 7);
   // columns of the two outer layers along x or z hold only shell voxels
   const bool              live = i >= 2 && i <= nx - 3 && k >= 2 && k <= nz - 3;
   const float             cx = 0.5f * float(nx - 1), cy = 0.5f * float(ny - 1), cz = 0.5f * float(nz - 1);
