@@ -8,7 +8,7 @@
 // Design (CDNA4):
 //  * Circular geometries make the detector column u and the perspective w
 //    independent of the volume y index (RTK's "OptimizedBackprojectionY" case).
-//    Each thread owns a column of NJ voxels (16, in small volumes 8) along y at fixed (x, z) and keeps
+//    Each thread owns a column of NJ voxels (16, in small volumes fewer) along y at fixed (x, z) and keeps
 //    them in registers for the whole launch; per view it computes u, w and the
 //    row step once (one reciprocal) and then only steps v along the column.
 //  * A workgroup is 16 (x) x 16 (z) such columns.  Per view it stages the detector
@@ -56,7 +56,7 @@ constexpr int kTileU = 64, kTileStride = 76; // staged detector footprint, pixel
 constexpr int
 TileRows(int NJ)
 {
-  return NJ == 8 ? 32 : 48;
+  return NJ == 16 ? 48 : 32;
 }
 constexpr int kPlaceViews = 64;                            // footprints placed per chunk, one per lane
 // A footprint whose every tap lies at least kEdge pixels inside the detector's
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
                                                      const float * vol_in, float * vol_out, int nx, int ny, int nz,
                                                      float ci, float cj, float ck)
 {
-  static_assert(NJ == 8 || NJ == 16, "a block is 16 heights or half of them");
+  static_assert(16 % NJ == 0, "a block is 16 heights or a part of them");
   constexpr int kTileV = TileRows(NJ), kStagePasses = kTileV / 16;
   __shared__ __align__(16) float stage[2][kTileV * kTileStride];
   __shared__ int4  rects[2][kPlaceViews]; // footprints (u0, v0, W, H) of two chunks of views
@@ -626,12 +626,23 @@ struct CoefCache
 };
 thread_local CoefCache g_cache;
 
-// Heights per block: 16, or 8 where 16 would give fewer workgroups than two rounds of the chip
-// (5 a CU).  A block of 8 stages and sets up as much per view for half the updates, but
-// small volumes leave the chip waiting: 128^3 <- 180 x 256^2 has 512 workgroups of 16.
-// 16 against 8: FDK of 128^3 <- 180 x 256^2 0.49 / 0.40 ms, of 203 x 181 x 221 (tilted, 2184
-// workgroups) 2.10 / 1.96, BP of 256^3 (4096) 2.58 either way, FDK of 512^3 40.0 / 42.8.
-constexpr long kSmallGrid = 2560;
+// Heights per block: 16, or fewer where that leaves the chip waiting.  A block of half the
+// heights stages and sets up as much per view for half the updates, but gives twice the
+// workgroups.  16 needs two rounds of the chip (5 workgroups a CU), 8 four workgroups a CU, 4 two.
+// Heights 16 / 8 / 4 / 2, ms, all else equal:
+//   FDK of 512^3 <- 720 x 1024^2 (32768 workgroups of 16)             40.0 / 42.8 / 54.5
+//   FDK of 203 x 181 x 221 <- 157, tilted (2184)                      2.10 / 1.96 / 1.96
+//   FDK of 128^3 <- 180 x 256^2 (512)                                 0.49 / 0.40 / 0.42
+//   2 x BP in CG of 119 x 88 x 104 <- 187, tilted (336)                    / 1.69 / 1.39 / 1.54
+//   FDK of 118 x 94 x 117 <- 97 x 160 x 128 (384)                          / .308 / .298 / .363
+//   FDK of 72 x 69 x 61 <- 289 x 112^2 (100)                               / .739 / .605 / .485
+//   FDK of 78 x 47 x 68 <- 319 x 96 x 80, tilted (75)                      / .993 / .699 / .585
+int
+BlockHeights(long columns, int ny)
+{
+  auto groups = [&](int NJ) { return columns * ((ny + NJ - 1) / NJ); };
+  return groups(16) >= 2560 ? 16 : groups(8) >= 1024 ? 8 : groups(4) >= 512 ? 4 : 2;
+}
 
 template <typename TP, bool FDK>
 void
@@ -640,7 +651,7 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
 {
   const TP * p = static_cast<const TP *>(proj);
   const long columns = long((nx + 15) / 16) * ((nz + 15) / 16);
-  const int  NJ = columns * ((ny + 15) / 16) < kSmallGrid ? 8 : 16;
+  const int  NJ = BlockHeights(columns, ny);
   dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + NJ - 1) / NJ);
   if (!column)
     grid = dim3(grid.x * grid.y * grid.z);
@@ -652,7 +663,9 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
                        ck);
   };
 #define RTKHIP_BP(VV, TT)                                                                                            \
-  NJ == 8 ? launch(bp_lds_kernel<TP, FDK, 8, VV, TT>) : launch(bp_lds_kernel<TP, FDK, 16, VV, TT>)
+  NJ == 16 ? launch(bp_lds_kernel<TP, FDK, 16, VV, TT>)                                                              \
+           : NJ == 8 ? launch(bp_lds_kernel<TP, FDK, 8, VV, TT>)                                                     \
+                     : NJ == 4 ? launch(bp_lds_kernel<TP, FDK, 4, VV, TT>) : launch(bp_lds_kernel<TP, FDK, 2, VV, TT>)
   if (column && vec)
     RTKHIP_BP(true, false);
   else if (column)

@@ -1,5 +1,5 @@
-"""Voxel and FDK backprojection by blocks of 8 heights (small volumes) and of 16 (from 2560
-blocks of 16^3), at the edges of both, with footprints inside the detector, across its border
+"""Voxel and FDK backprojection by blocks of 2, 4, 8 (small volumes) and 16 heights (from 2560
+blocks of 16^3), at their edges, with footprints inside the detector, across its border
 and outside it, against the float oracle with the backprojector's bar of 1e-5 relative L2."""
 import numpy as np
 import pytest
@@ -9,7 +9,8 @@ from helpers import hip_geometry, rel_l2, to_device
 pytestmark = pytest.mark.gpu
 
 SMALL = [(40, ny, 33) for ny in (1, 7, 8, 9, 16, 23, 24, 25, 47)]
-LARGE = [(330, 95, 335), (330, 97, 335), (330, 80, 335)]  # 6, 7 and 5 blocks of 21 x 21
+# 6, 7 and 5 blocks of 16 heights by 21 x 21 columns of them; 8 blocks of 8 by 11 x 11
+LARGE = [(330, 95, 335), (330, 97, 335), (330, 80, 335), (170, 59, 171), (170, 61, 171)]
 
 
 def _run(oracle, hip, vsize, fdk, stack):
