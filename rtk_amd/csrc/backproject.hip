@@ -232,11 +232,11 @@ ItkLinear(const TP * pp, int nu, int nv, float tu, float tv)
   return vx0 + (vx1 - vx0) * d1;
 }
 
-// One voxel of one view, read from global memory: per-voxel perspective, per-view border
-// rule.
+// One voxel of one view added to acc, read from global memory: per-voxel perspective,
+// per-view border rule.
 template <typename TP, bool FDK>
 __device__ __forceinline__ float
-UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float x, float y, float z)
+UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float x, float y, float z, float acc)
 {
   // written out, so that every caller rounds alike: one ulp of u or v can decide whether
   // a voxel is inside the border
@@ -246,8 +246,8 @@ UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float
   {
     // Inside iff -0.5 <= idx < n - 0.5 in both directions.
     if (v >= -0.5f && v < float(nv) - 0.5f && u >= -0.5f && u < float(nu) - 0.5f)
-      return (FDK ? rw * rw : 1.f) * ItkLinear(pp, nu, nv, v, u);
-    return 0.f;
+      return fmaf(FDK ? rw * rw : 1.f, ItkLinear(pp, nu, nv, v, u), acc);
+    return acc;
   }
   const float uf = floorf(u), vf = floorf(v);
   if (uf >= 0.f && int(uf) < nu - 1 && vf >= 0.f && int(vf) < nv - 1)
@@ -258,9 +258,9 @@ UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float
     const float a = LoadPix(pp, o), b = LoadPix(pp, o + nu), cc = LoadPix(pp, o + 1), d = LoadPix(pp, o + nu + 1);
     const float t0 = (1.f - fv) * a + fv * b;
     const float t1 = (1.f - fv) * cc + fv * d;
-    return (FDK ? rw * rw : 1.f) * ((1.f - fu) * t0 + fu * t1);
+    return fmaf(FDK ? rw * rw : 1.f, (1.f - fu) * t0 + fu * t1, acc);
   }
-  return 0.f;
+  return acc;
 }
 
 // TILT: the views' u and w may depend on y and their border rule may be ITK's (border[p],
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
         for (int jj = 0; jj < NJ; jj++)
         {
           const float first =
-            acc[0] + (jj < jn ? UpdateGeneral<TP, FDK>(c, itk, pp, nu, nv, x, y0 + float(jj), z) : 0.f);
+            jj < jn ? UpdateGeneral<TP, FDK>(c, itk, pp, nu, nv, x, y0 + float(jj), z, acc[0]) : acc[0];
 #pragma unroll
           for (int q = 0; q + 1 < NJ; q++)
             acc[q] = acc[q + 1];
@@ -618,6 +618,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
   }
 }
 
+// The smallest tilted volumes, a thread per voxel: too few for blocks, whose views follow each
+// other behind a barrier each, and a stack that the L2s hold.  Same sums as the blocks'.
+// Blocks / per voxel, whole calls, ms: FDK 84 x 72 x 76 <- 249 .66 / .40, 92 x 60 x 89 <- 274
+// .65 / .50; CG 91 x 86 x 80 <- 73 .62 / .57; FDK 93 x 82 x 90 <- 294 .73 / .76, 124 x 76 x
+// 109 <- 119 .49 / .54.
+constexpr long kPerVoxel = 640L << 10;
+template <typename TP, bool FDK>
+__global__ __launch_bounds__(256) void bp_voxel_kernel(const ViewCoef * __restrict__ views,
+                                                       const int * __restrict__ border, int nviews,
+                                                       const TP * __restrict__ proj, int nu, int nv,
+                                                       const float * vol_in, float * vol_out, int nx, int ny, int nz,
+                                                       float ci, float cj, float ck)
+{
+  const int idx = int(blockIdx.x * blockDim.x + threadIdx.x);
+  if (idx >= nx * ny * nz)
+    return;
+  const int   row = idx / nx;
+  const float x = float(idx - row * nx) - ci, y = float(row % ny) - cj, z = float(row / ny) - ck;
+  float       acc = vol_in ? vol_in[idx] : 0.f;
+  for (int p = 0; p < nviews; p++)
+    acc = UpdateGeneral<TP, FDK>(views[p], border && border[p] == RTKHIP_BORDER_ITK_LINEAR,
+                                 proj + long(p) * (long(nu) * nv), nu, nv, x, y, z, acc);
+  vol_out[idx] = acc;
+}
+
 // Per-(thread, stream) cache of the uploaded view coefficients.
 struct CoefCache
 {
@@ -636,7 +661,7 @@ thread_local CoefCache g_cache;
 //   2 x BP in CG of 119 x 88 x 104 <- 187, tilted (336)                    / 1.69 / 1.39 / 1.54
 //   FDK of 118 x 94 x 117 <- 97 x 160 x 128 (384)                          / .308 / .298 / .363
 //   FDK of 72 x 69 x 61 <- 289 x 112^2 (100)                               / .739 / .605 / .485
-//   FDK of 78 x 47 x 68 <- 319 x 96 x 80, tilted (75)                      / .993 / .699 / .585
+// (Tilted volumes of 2 go voxel by voxel, kPerVoxel.)
 int
 BlockHeights(long columns, int ny)
 {
@@ -650,6 +675,14 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
        const float * vin, float * vout, int nx, int ny, int nz, float ci, float cj, float ck, hipStream_t s)
 {
   const TP * p = static_cast<const TP *>(proj);
+  const long vox = long(nx) * ny * nz;
+  if (!column && vox < kPerVoxel)
+  {
+    hipLaunchKernelGGL((bp_voxel_kernel<TP, FDK>), dim3(unsigned((vox + 255) / 256)), dim3(256), 0, s, dcoef, dborder,
+                       nviews, p, nu, nv, vin, vout, nx, ny, nz, ci, cj, ck);
+    RTKHIP_CHECK_LAUNCH();
+    return;
+  }
   const long columns = long((nx + 15) / 16) * ((nz + 15) / 16);
   const int  NJ = BlockHeights(columns, ny);
   dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + NJ - 1) / NJ);
@@ -665,7 +698,7 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
 #define RTKHIP_BP(VV, TT)                                                                                            \
   NJ == 16 ? launch(bp_lds_kernel<TP, FDK, 16, VV, TT>)                                                              \
            : NJ == 8 ? launch(bp_lds_kernel<TP, FDK, 8, VV, TT>)                                                     \
-                     : NJ == 4 ? launch(bp_lds_kernel<TP, FDK, 4, VV, TT>) : launch(bp_lds_kernel<TP, FDK, 2, VV, TT>)
+                     : NJ == 4 ? launch(bp_lds_kernel<TP, FDK, 4, VV, TT>) : launch(bp_lds_kernel<TP, FDK, TT ? 4 : 2, VV, TT>)
   if (column && vec)
     RTKHIP_BP(true, false);
   else if (column)
