@@ -1925,8 +1925,8 @@ struct GatherPlan
 {
   std::vector<GatherView>   views;
   std::vector<GatherColumn> cols;
-  std::vector<signed char>  axis;
-  std::vector<int>          single; // columns (view * nu + iu) of no single axis, taken ray by ray
+  std::vector<signed char>  axis;   // the backprojector's axis per column, then the forward projector's
+  std::vector<int>          single; // columns (view * nu + iu) the forward projector takes ray by ray
   std::vector<int>          blocks; // packed block coordinates (bx | bz << 10 | by << 20)
   int                       freeRows = 1; // leading candidate rows whose weight needs no clamp
   double                    maxRowStep = 0.; // largest height step between adjacent rows inside the volume
@@ -1951,7 +1951,7 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
   const double ctr[3] = { cx, cy, cz };
   G.views.assign(np, GatherView{});
   G.cols.assign(size_t(np) * nu, GatherColumn{});
-  G.axis.assign(size_t(np) * nu, -1);
+  G.axis.assign(2 * size_t(np) * nu, -1);
   double minRowStep = DBL_MAX, maxRowStep = 0.;
   for (int p = 0; p < np; p++)
   {
@@ -1998,18 +1998,19 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
     {
       const double px = o[0] + iu * eu[0], pz = o[2] + iu * eu[2];
       const double dx = S[0] - px, dz = S[2] - pz;
-      // a margin keeps the columns whose dominant axis rounding decides out of the tables
+      // The forward projector takes a ray's axis from its column, so a margin leaves the
+      // columns whose axis rounding decides to the kernel that sets every ray up.  The
+      // backprojector's per-ray pass does that for every ray (one of another axis than its
+      // column's is splatted), so it needs no margin, and a column on a diagonal is gathered
+      // like any other: by atomics its sums would change from run to run.
       constexpr double kTie = 1. + 1e-9;
-      int              ax = -1;
-      if (std::abs(dx) > kTie * std::abs(dz) && std::abs(dx) > kTie * mh)
-        ax = 0;
-      else if (std::abs(dz) > kTie * std::abs(dx) && std::abs(dz) > kTie * mh)
-        ax = 2;
-      if (ax < 0)
-      {
+      const double     adx = std::abs(dx), adz = std::abs(dz);
+      const int        ax = adx >= adz && adx >= mh ? 0 : (adz > adx && adz > mh ? 2 : -1);
+      const bool       clear = std::max(adx, adz) > kTie * std::min(adx, adz) && std::max(adx, adz) > kTie * mh;
+      if (ax < 0 || !clear)
         G.single.push_back(p * nu + iu);
+      if (ax < 0)
         continue;
-      }
       GatherColumn & C = G.cols[size_t(p) * nu + iu];
       const double   dk = ax == 0 ? dx : dz, dh = ax == 0 ? dz : dx;
       const double   pk = ax == 0 ? px : pz, ph = ax == 0 ? pz : px;
@@ -2046,6 +2047,8 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
         maxRowStep = std::max(maxRowStep, std::abs(ev[1] * (1. - tIn)));
       }
       G.axis[size_t(p) * nu + iu] = static_cast<signed char>(ax);
+      if (clear)
+        G.axis[(size_t(np) + p) * nu + iu] = static_cast<signed char>(ax);
       (ax == 0 ? V.hasX : V.hasZ) = 1;
     }
   }
@@ -2103,7 +2106,7 @@ PrepareGather(const int proj_dim[3], const int vol_dim[3], const double * proj_t
     auto & gb = g_joseph.gblocks[s];
     gv.Resize(np);
     gc.Resize(size_t(np) * nu);
-    ga.Resize(size_t(np) * nu);
+    ga.Resize(G.axis.size());
     gb.Resize(G.blocks.size());
     RTKHIP_CHECK(hipMemcpyAsync(gv.get(), G.views.data(), sizeof(GatherView) * np, hipMemcpyHostToDevice, s));
     RTKHIP_CHECK(hipMemcpyAsync(gc.get(), G.cols.data(), sizeof(GatherColumn) * G.cols.size(),
@@ -2356,9 +2359,9 @@ rtkhip_joseph_forward_project(const int proj_dim[3], const int vol_dim[3], const
 #define RTKHIP_FCOL(WW, QQ, EE)                                                                                      \
   if (shape.w == WW && shape.q == QQ && shape.e == EE)                                                               \
     hipLaunchKernelGGL((joseph_fp_column_kernel<WW, QQ, EE>), fg, dim3(64 * WW), 0, s, g_joseph.gviews[s].get(),     \
-                       g_joseph.gcols[s].get(), g_joseph.gaxis[s].get(), nu, nv, dev_proj_in, dev_proj_out,          \
-                       dT.get() + 1, int(pitch), vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1], \
-                       vol_spacing[2], xcdOrder);
+                       g_joseph.gcols[s].get(), g_joseph.gaxis[s].get() + size_t(np) * nu, nu, nv, dev_proj_in,      \
+                       dev_proj_out, dT.get() + 1, int(pitch), vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0],   \
+                       vol_spacing[1], vol_spacing[2], xcdOrder);
         RTKHIP_COLUMN_SHAPES(RTKHIP_FCOL)
 #undef RTKHIP_FCOL
         if (const int n = g_joseph.gplanSingle[s])
