@@ -930,7 +930,8 @@ struct GatherView
   float  pu[4], pv[4], pw[4]; // centred volume index (x', y', z', 1) -> detector (u w, v w, w)
   double y0, y1, sy;          // y' of row jv at depth t: (y0 + y1 jv)(1 - t) + sy t
   int    hasX, hasZ;          // columns walking along x / along z exist in this view
-  int    pad[2];
+  int    faceRow;             // row whose rays run along a face of the volume (-1: none)
+  int    pad;
 };
 
 struct GatherColumn
@@ -1468,7 +1469,8 @@ struct ColumnPath
   double x0, h1, t0, t1, near, far;
 };
 
-// Narrows [near, far] to where p0 + k slope lies in [0, last].
+// Narrows [near, far] to where p0 + k slope lies in [0, last].  SetupRay's box ends a rounding
+// short of last, which only shows for rays that run along a face: those are not taken here.
 __device__ __forceinline__ void
 ClipPath(double p0, double slope, double last, double & near, double & far)
 {
@@ -1546,9 +1548,11 @@ EndSample(const ColumnPath & P, const ColumnRay & R, int k, double step, const f
   return float(double(r) * step);
 }
 
-// Rays of the columns the sweep does not take (they mix dominant axes, or lie so close to
-// a change of axis that rounding decides it), one ray per thread, as the per-ray forward
-// projector walks them.  columns: view * nu + iu.
+// Rays that the sweep does not take, one per thread, as the per-ray forward projector walks
+// them: columns (lines[blockIdx.x] = view * nu + iu) that mix dominant axes, lie so close to a
+// change of axis that rounding decides it, or run along a face of the volume, where SetupRay's
+// rounding decides whether a ray hits at all; and (ROW) the view lines[blockIdx.x]'s faceRow,
+// in the columns that the sweep takes.
 __device__ __forceinline__ float
 RayBorder(const Ray & R, const ColumnStrides & S, double step, const float * slice, double x, double y)
 {
@@ -1562,15 +1566,16 @@ RayBorder(const Ray & R, const ColumnStrides & S, double step, const float * sli
   return float(double(r) * step);
 }
 
-__global__ __launch_bounds__(64) void joseph_fp_single_kernel(const JosephView * __restrict__ views,
-                                                               const int * __restrict__ columns, int nu, int nv,
-                                                               const float * pin, float * pout,
-                                                               const float * __restrict__ vol, int pitch, int nx,
-                                                               int ny, int nz, double spx, double spy, double spz,
-                                                               double infClip, double supClip)
+template <bool ROW>
+__global__ __launch_bounds__(64) void joseph_fp_single_kernel(
+  const JosephView * __restrict__ views, const GatherView * __restrict__ gviews,
+  const signed char * __restrict__ colAxis, const int * __restrict__ lines, int nu, int nv, const float * pin,
+  float * pout, const float * __restrict__ vol, int pitch, int nx, int ny, int nz, double spx, double spy, double spz,
+  double infClip, double supClip)
 {
-  const int p = columns[blockIdx.x] / nu, iu = columns[blockIdx.x] % nu, jv = blockIdx.y * 64 + threadIdx.x;
-  if (jv >= nv)
+  const int line = lines[blockIdx.x], along = blockIdx.y * 64 + threadIdx.x;
+  const int p = ROW ? line : line / nu, iu = ROW ? along : line % nu, jv = ROW ? gviews[p].faceRow : along;
+  if (along >= (ROW ? nu : nv) || (ROW && colAxis[size_t(p) * nu + iu] < 0))
     return;
   const size_t pix = (size_t(p) * nv + jv) * nu + iu;
   const float  base = pin ? pin[pix] : 0.f;
@@ -1875,7 +1880,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(Q <= 2 ?
   for (int q = 0; q < Q; q++)
   {
     const int jv = r0 + lane + 64 * q;
-    if (jv >= nv)
+    if (jv >= nv || jv == V.faceRow)
       continue;
     const ColumnRay R = RayOf(V, P, jv, ny);
     const size_t    pix = (size_t(p) * nv + jv) * nu + iu;
@@ -1915,8 +1920,9 @@ struct JosephCache
   std::map<hipStream_t, std::vector<double>> gplanKey;
   std::map<hipStream_t, long long>           gplanBlocks; // -1: the gather does not apply
   std::map<hipStream_t, int>                 gplanFree;
-  std::map<hipStream_t, int>                        gplanSingle; // entries of gsingle
-  std::map<hipStream_t, double>                     gplanRowStep;
+  std::map<hipStream_t, int>                 gplanSingle; // columns of gsingle
+  std::map<hipStream_t, int>                 gplanFaces;  // views with a faceRow, after them in gsingle
+  std::map<hipStream_t, double>              gplanRowStep;
 };
 thread_local JosephCache g_joseph;
 
@@ -1927,6 +1933,7 @@ struct GatherPlan
   std::vector<GatherColumn> cols;
   std::vector<signed char>  axis;   // the backprojector's axis per column, then the forward projector's
   std::vector<int>          single; // columns (view * nu + iu) the forward projector takes ray by ray
+  std::vector<int>          faces;  // views that have a faceRow
   std::vector<int>          blocks; // packed block coordinates (bx | bz << 10 | by << 20)
   int                       freeRows = 1; // leading candidate rows whose weight needs no clamp
   double                    maxRowStep = 0.; // largest height step between adjacent rows inside the volume
@@ -1994,19 +2001,33 @@ PlanGather(const int proj_dim[3], const int vol_dim[3], const double * proj_to_v
     V.sy = S[1] - cy;
     const double dyTop = std::abs(S[1] - o[1]), dyBot = std::abs(S[1] - (o[1] + (nv - 1) * ev[1]));
     const double mh = std::max(dyTop, dyBot);
+    // Rays that stay within kFace of a face's plane along the whole of their path, of which
+    // rounding (at most 1e-11 of a position) decides whether they hit: the row at the source's
+    // height, if a face is there.
+    // The place where a steeper ray of n slices crosses a face's plane moves by 1e-7 n slices.
+    constexpr double kFace = 1e-4;
+    auto             onFace = [](double a, double b, int n) {
+      return std::abs(a - b) < kFace && std::min(std::abs(a), std::abs(a - (n - 1))) < kFace;
+    };
+    const double js = std::round((S[1] - o[1]) / ev[1]);
+    V.faceRow = js >= 0. && js < nv && onFace(S[1], o[1] + js * ev[1], ny) ? int(js) : -1;
+    if (V.faceRow >= 0)
+      G.faces.push_back(p);
     for (int iu = 0; iu < nu; iu++)
     {
       const double px = o[0] + iu * eu[0], pz = o[2] + iu * eu[2];
       const double dx = S[0] - px, dz = S[2] - pz;
       // The forward projector takes a ray's axis from its column, so a margin leaves the
-      // columns whose axis rounding decides to the kernel that sets every ray up.  The
+      // columns whose axis rounding decides to the kernel that sets every ray up, as those
+      // along a face.  The
       // backprojector's per-ray pass does that for every ray (one of another axis than its
       // column's is splatted), so it needs no margin, and a column on a diagonal is gathered
       // like any other: by atomics its sums would change from run to run.
       constexpr double kTie = 1. + 1e-9;
       const double     adx = std::abs(dx), adz = std::abs(dz);
       const int        ax = adx >= adz && adx >= mh ? 0 : (adz > adx && adz > mh ? 2 : -1);
-      const bool       clear = std::max(adx, adz) > kTie * std::min(adx, adz) && std::max(adx, adz) > kTie * mh;
+      const bool       face = onFace(S[0], px, nx) || onFace(S[2], pz, nz);
+      const bool       clear = !face && std::max(adx, adz) > kTie * std::min(adx, adz) && std::max(adx, adz) > kTie * mh;
       if (ax < 0 || !clear)
         G.single.push_back(p * nu + iu);
       if (ax < 0)
@@ -2114,16 +2135,18 @@ PrepareGather(const int proj_dim[3], const int vol_dim[3], const double * proj_t
     RTKHIP_CHECK(hipMemcpyAsync(ga.get(), G.axis.data(), G.axis.size(), hipMemcpyHostToDevice, s));
     RTKHIP_CHECK(
       hipMemcpyAsync(gb.get(), G.blocks.data(), sizeof(int) * G.blocks.size(), hipMemcpyHostToDevice, s));
-    if (!G.single.empty())
+    std::vector<int> lines = G.single;
+    lines.insert(lines.end(), G.faces.begin(), G.faces.end());
+    if (!lines.empty())
     {
       auto & gs = g_joseph.gsingle[s];
-      gs.Resize(G.single.size());
-      RTKHIP_CHECK(
-        hipMemcpyAsync(gs.get(), G.single.data(), sizeof(int) * G.single.size(), hipMemcpyHostToDevice, s));
+      gs.Resize(lines.size());
+      RTKHIP_CHECK(hipMemcpyAsync(gs.get(), lines.data(), sizeof(int) * lines.size(), hipMemcpyHostToDevice, s));
     }
     nblocks = (long long)G.blocks.size();
   }
   g_joseph.gplanSingle[s] = int(G.single.size());
+  g_joseph.gplanFaces[s] = int(G.faces.size());
   g_joseph.gplanBlocks[s] = nblocks;
   g_joseph.gplanFree[s] = freeRows = G.freeRows;
   g_joseph.gplanRowStep[s] = G.maxRowStep;
@@ -2364,14 +2387,18 @@ rtkhip_joseph_forward_project(const int proj_dim[3], const int vol_dim[3], const
                        vol_spacing[1], vol_spacing[2], xcdOrder);
         RTKHIP_COLUMN_SHAPES(RTKHIP_FCOL)
 #undef RTKHIP_FCOL
-        if (const int n = g_joseph.gplanSingle[s])
-        {
+        const int nsingle = g_joseph.gplanSingle[s], nfaces = g_joseph.gplanFaces[s];
+        auto      single = [&](auto kernel, const int * lines, int n, int along) {
           RTKHIP_CHECK_LAUNCH();
-          hipLaunchKernelGGL(joseph_fp_single_kernel, dim3(unsigned(n), unsigned((nv + 63) / 64)), dim3(64), 0, s, dv,
-                             g_joseph.gsingle[s].get(), nu, nv, dev_proj_in, dev_proj_out, dT.get() + 1, int(pitch),
-                             vol_dim[0], vol_dim[1], vol_dim[2], vol_spacing[0], vol_spacing[1], vol_spacing[2],
-                             infClip, supClip);
-        }
+          hipLaunchKernelGGL(kernel, dim3(unsigned(n), unsigned((along + 63) / 64)), dim3(64), 0, s, dv,
+                             g_joseph.gviews[s].get(), g_joseph.gaxis[s].get() + size_t(np) * nu, lines, nu, nv,
+                             dev_proj_in, dev_proj_out, dT.get() + 1, int(pitch), vol_dim[0], vol_dim[1], vol_dim[2],
+                             vol_spacing[0], vol_spacing[1], vol_spacing[2], infClip, supClip);
+        };
+        if (nsingle)
+          single(joseph_fp_single_kernel<false>, g_joseph.gsingle[s].get(), nsingle, nv);
+        if (nfaces)
+          single(joseph_fp_single_kernel<true>, g_joseph.gsingle[s].get() + nsingle, nfaces, nu);
       }
       else
       {
