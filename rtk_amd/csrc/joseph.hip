@@ -31,7 +31,6 @@
 
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
-#include <array>
 #include <cfloat>
 #include <climits>
 #include <cmath>
@@ -1335,8 +1334,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
   }
 }
 
+// Columns of the two outer layers along x and along z.
+__host__ __device__ __forceinline__ int
+ShellColumns(int nx, int nz)
+{
+  return 4 * (nx + nz - 4);
+}
+
+// Column c of them, in an order in which neighbours of a face follow each other (their
+// candidate rays overlap): the layers z = 0, 1, nz - 2, nz - 1, then, without those, the
+// layers x = 0, 1, nx - 2, nx - 1.
+__device__ __forceinline__ void
+ShellColumn(int c, int nx, int nz, int & i, int & k)
+{
+  auto      layer = [](int q, int n) { return q < 2 ? q : n - 4 + q; };
+  const int d = c - 4 * nx;
+  k = d < 0 ? layer(c / nx, nz) : 2 + d % (nz - 4);
+  i = d < 0 ? c % nx : layer(d / (nz - 4), nx);
+}
+
 // The voxels of the two outer layers along x and along z: a wavefront is 64 heights of one of
-// their columns (indices k nx + i from `shell`), reading the rays from global memory.  These
+// their columns, reading the rays from global memory.  These
 // voxels also receive first and last steps, so each candidate (ray, slice) takes its step
 // weight from the ray's first/last slices and, on those, its position clamped into the box.
 // The candidate columns are the same for all 64 heights (scalar loop and table reads), and
@@ -1347,7 +1365,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void j
 __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
   const GatherView * __restrict__ gviews, const GatherColumn * __restrict__ gcols,
   const signed char * __restrict__ colAxis, int nviews, int nu, int nv, const uint2 * __restrict__ gend,
-  const float2 * __restrict__ gw, const int * __restrict__ shell, int ncolumns, float * vol, int nx, int ny, int nz)
+  const float2 * __restrict__ gw, float * vol, int nx, int ny, int nz)
 {
   // Workgroups are dealt to the 8 XCDs in turn; XCD x takes a contiguous run of the
   // columns instead of every 8th workgroup, so the voxels one XCD's L2 serves lie
@@ -1355,10 +1373,11 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
   const unsigned nb = gridDim.x, full = nb / 8, rem = nb % 8, x = blockIdx.x % 8, q = blockIdx.x / 8;
   const unsigned lb = x * full + min(x, rem) + q;
   const unsigned bands = (ny + 63) / 64, w = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (w >= unsigned(ncolumns) * bands)
+  if (w >= unsigned(ShellColumns(nx, nz)) * bands)
     return;
-  const int    column = __builtin_amdgcn_readfirstlane(shell[w / bands]);
-  const int    i = column % nx, j = int(w % bands) * 64 + int(threadIdx.x & 63), k = column / nx;
+  int          i, k;
+  ShellColumn(int(w / bands), nx, nz, i, k);
+  const int    j = int(w % bands) * 64 + int(threadIdx.x & 63);
   const float  cx = 0.5f * float(nx - 1), cy = 0.5f * float(ny - 1), cz = 0.5f * float(nz - 1);
   const float  xc = float(i) - cx, zc = float(k) - cz, yv = float(j) - cy;
   const double xd = double(xc), zd = double(zc);
@@ -1911,9 +1930,6 @@ struct JosephCache
   std::map<hipStream_t, DeviceBuffer<float>>        gval;
   std::map<hipStream_t, DeviceBuffer<uint2>>        gend;
   std::map<hipStream_t, DeviceBuffer<float2>>       gw;
-  std::map<hipStream_t, DeviceBuffer<int>>          gshell; // columns of the outer layers along x and z
-  std::map<hipStream_t, std::array<int, 3>>         gshellDims;
-  std::map<hipStream_t, int>                        gshellCount;
   // the arguments the uploaded tables were made from: a call with the same ones (every
   // iteration of an iterative reconstruction) reuses them without host work or copies
   std::map<hipStream_t, std::vector<double>> viewsKey;
@@ -2167,25 +2183,6 @@ GatherBackproject(long long nblocks, int freeRows, const JosephView * dv, const 
   auto &    gc = g_joseph.gcols[s];
   auto &    ga = g_joseph.gaxis[s];
   auto &    gb = g_joseph.gblocks[s];
-  // the columns of the two outer layers along x and z, listed once per volume size
-  auto &                   gs = g_joseph.gshell[s];
-  const std::array<int, 3> dims = { nx, ny, nz };
-  if (!gs.get() || g_joseph.gshellDims[s] != dims)
-  {
-    // neighbouring columns of a face follow each other: their candidate rays overlap
-    std::vector<int> shell;
-    for (int z : { 0, 1, nz - 2, nz - 1 })
-      for (int x = 0; x < nx; x++)
-        shell.push_back(z * nx + x);
-    for (int x : { 0, 1, nx - 2, nx - 1 })
-      for (int z = 2; z < nz - 2; z++)
-        shell.push_back(z * nx + x);
-    gs.Resize(shell.size());
-    RTKHIP_CHECK(hipMemcpy(gs.get(), shell.data(), sizeof(int) * shell.size(), hipMemcpyHostToDevice));
-    g_joseph.gshellDims[s] = dims;
-    g_joseph.gshellCount[s] = int(shell.size());
-  }
-  const int nshell = g_joseph.gshellCount[s];
   const size_t rays = size_t(nu) * nv;
   const int    chunk = int(std::max<size_t>(1, std::min<size_t>(np, (size_t(1) << 30) / (20 * rays))));
   auto &       dval = g_joseph.gval[s];
@@ -2214,10 +2211,10 @@ GatherBackproject(long long nblocks, int freeRows, const JosephView * dv, const 
                        dim3(256), 0, s, gv.get() + p0, gc.get() + size_t(p0) * nu, ga.get() + size_t(p0) * nu, c, nu,
                        nv, dval.get(), dend.get(), dw.get(), gb.get(), vol, nx, ny, nz);
     RTKHIP_CHECK_LAUNCH();
-    const long shellWaves = long(nshell) * ((ny + 63) / 64);
+    const long shellWaves = long(ShellColumns(nx, nz)) * ((ny + 63) / 64);
     hipLaunchKernelGGL(joseph_gather_shell_kernel, dim3(unsigned((shellWaves + 3) / 4)), dim3(256), 0, s,
                        gv.get() + p0, gc.get() + size_t(p0) * nu, ga.get() + size_t(p0) * nu, c, nu, nv, dend.get(),
-                       dw.get(), gs.get(), nshell, vol, nx, ny, nz);
+                       dw.get(), vol, nx, ny, nz);
     RTKHIP_CHECK_LAUNCH();
   }
 }
