@@ -26,6 +26,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <type_traits>
@@ -684,7 +685,9 @@ Launch(bool column, const ViewCoef * dcoef, const int * dborder, int nviews, con
     return;
   }
   const long columns = long((nx + 15) / 16) * ((nz + 15) / 16);
-  const int  NJ = BlockHeights(columns, ny);
+  // one value for the grid and the kernel; the TILT form has no blocks of 2 (volumes of fewer
+  // voxels than kPerVoxel take none)
+  const int  NJ = std::max(BlockHeights(columns, ny), column ? 2 : 4);
   dim3       grid((nx + 15) / 16, (nz + 15) / 16, (ny + NJ - 1) / NJ);
   if (!column)
     grid = dim3(grid.x * grid.y * grid.z);
