@@ -325,7 +325,7 @@ struct Walker
   {
     int cix, ciy;
     Stage2D(R, cix, ciy, lx, ly);
-    return cix + int(__umul24(unsigned(ciy), unsigned(R.oy)));
+    return cix + ciy * R.oy; // 32 bits: a z row of a y-dominant ray may be 2^24 voxels and more
   }
   // Lower-left tap (cix, ciy) of the current sample, then advance one slice.
   __device__ __forceinline__ void Stage2D(const Ray & R, int & cix, int & ciy, float & lx, float & ly)
@@ -419,18 +419,18 @@ __global__ __launch_bounds__(256) void joseph_kernel(const JosephView * __restri
     const int     t0 = lock ? (R.ns - kfirst) * dirSign : INT_MAX;
     const int     tEnd = lock ? t0 + R.nmid + 1 : INT_MIN; // R.nmid = -1 when fs == ns
     Walker        wk;
+    const unsigned oy = unsigned(axis == 0 ? nz : (axis == 1 ? nx * ny : nx)); // R.oy of the locked rays
     // a ray whose first and last middle samples lie inside the slice needs no index clamp;
     // byte offsets within a slice fit 32 bits (below 2^31 voxels in at least two slices; a
-    // slice along y spans the volume)
+    // slice along y spans the volume) and their products 24-bit factors
     bool free = false;
-    if (lock && R.nmid > 0 && (axis != 1 || long(nx) * ny * nz < (1L << 30)))
+    if (lock && R.nmid > 0 && oy < (1u << 24) && (axis != 1 || long(nx) * ny * nz < (1L << 30)))
     {
       wk.Init(R.cx + R.stepx, R.cy + R.stepy);
       const long long X1 = wk.X + (R.nmid - 1) * R.sx32, Y1 = wk.Y + (R.nmid - 1) * R.sy32;
       free = wk.X >= 0 && X1 >= 0 && int(wk.X >> 32) <= R.nxm2 && int(X1 >> 32) <= R.nxm2 && wk.Y >= 0 && Y1 >= 0 &&
              int(wk.Y >> 32) <= R.nym2 && int(Y1 >> 32) <= R.nym2;
     }
-    const unsigned oy = unsigned(axis == 0 ? nz : (axis == 1 ? nx * ny : nx)); // R.oy of the locked rays
     const long step = dirSign * absOz;
     for (int s = 0; s < nsl; s += kLockBatch)
     {
