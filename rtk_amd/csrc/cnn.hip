@@ -245,17 +245,31 @@ __global__ __launch_bounds__(256, 2) void conv32_mfma_kernel(const bf16_t * __re
 }
 
 // ------------------------------------------------------------------ layer 6
+
+// Whether one of eight activations (ReLU outputs: the order of the values is that of their
+// bits) is infinite; a negative zero counts as one.
+__device__ __forceinline__ bool
+HasInf(const bf16x8 & v)
+{
+  typedef unsigned short ushort8v __attribute__((ext_vector_type(8)));
+  typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+  const ushort8v  b = __builtin_bit_cast(ushort8v, v);
+  const ushort2v  m = __builtin_elementwise_max(__builtin_elementwise_max(b.lo.lo, b.lo.hi),
+                                               __builtin_elementwise_max(b.hi.lo, b.hi.hi));
+  return max(m.x, m.y) >= 0x7f80;
+}
+
 // y[v] = x[v] + (b6 + sum_t sum_ci W6[t][ci] a5[v + d(t)][ci]) / s
 // As a GEMM per voxel u of the input, P[t][u] = sum_ci W6[t][ci] a5[u][ci] (M = 27 taps in two
 // halves of 16, N = 16 voxels, K = 32 channels), and the sum y[v] += P[t][v + d(t)].  The FP32
 // weights enter as three BF16 terms whose sum is the weight exactly (24 bits in three times
 // 8), so every product is exact and the sums are FP32; with fewer sequential additions y's
 // error against 64 bits is a quarter of the tap-by-tap loop's (1.2e-7 of the range, 4.8e-7
-// before).  (An infinite activation gives NaN: a weight's lower terms may be 0.)  A workgroup
-// is a 16 x 16 (x, y) column marching along z: per plane its wavefronts write P of the
-// 18 x 18 halo to LDS, then each thread adds 9 values to each of the three outputs the plane
-// feeds, which it keeps in registers; the next plane's activations are loaded meanwhile.
-// Every activation is read 1.3 times instead of 27.
+// before).  Infinite activations meet the weights' first terms alone: a lower term may be 0 or
+// of the other sign.  A workgroup is a 16 x 16 (x, y) column marching along z: per plane its
+// wavefronts write P of the 18 x 18 halo to LDS, then each thread adds 9 values to each of the
+// three outputs the plane feeds, which it keeps in registers; the next plane's activations are
+// loaded meanwhile.  Every activation is read 1.3 times instead of 27.
 // 256^3: 1.65 ms (864 VALU FMAs and 108 cached 16-byte loads a voxel) -> 0.27 ms.
 constexpr int kOutX = 16, kOutHX = kOutX + 2, kOutVox = kOutHX * kOutHX; // halo plane
 constexpr int kOutGroups = (kOutVox + 15) / 16;
@@ -319,13 +333,18 @@ __global__ __launch_bounds__(256) void conv_out_kernel(const bf16_t * __restrict
       const int v = 16 * (wave + 4 * g) + col;
       if (16 * (wave + 4 * g) >= kOutVox)
         continue; // uniform
+      bf16x8 low = act[g]; // for the weights' lower terms
+      if (__any(HasInf(low)))
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          low[e] = fabsf(float(low[e])) < INFINITY ? low[e] : bf16_t(0.f);
 #pragma unroll
       for (int h = 0; h < 2; h++)
       {
         floatx4 acc = floatx4{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
         for (int k = 2; k >= 0; k--)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[h][k], act[g], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[h][k], k ? low : act[g], acc, 0, 0, 0);
 #pragma unroll
         for (int q = 0; q < 4; q++)
           if (16 * h + 4 * kg + q < T)
