@@ -324,6 +324,12 @@ int rtkhip_forward_project(rtkhip_context * c, const rtkhip_geometry * g, const 
                            const float * dev_proj_in, float * dev_proj_out, const rtkhip_image * vol,
                            const float * dev_vol, long long * samples, void * stream);
 
+/* How rtkhip_forward_project takes these images, for tests and tuning: columns a workgroup,
+ * rows a lane and 64-height runs a profile of its kernel for vertical detector columns, or
+ * zeros where it goes ray by ray.  Host only. */
+int rtkhip_forward_project_shape(const rtkhip_geometry * g, const rtkhip_image * stack, const rtkhip_image * vol,
+                                 int shape[3]);
+
 /* rtk::HipBackProjectionImageFilter (voxel-based, fdk = 0) and the FDK
  * backprojector (fdk = 1).  vol_out = vol_in + BP(proj). */
 int rtkhip_back_project(rtkhip_context * c, const rtkhip_geometry * g, const rtkhip_image * vol,

@@ -86,6 +86,7 @@ SIGNATURES = [
     ("rtkhip_fft_ramp_filter", I, [P, ctypes.POINTER(Image), P, P, ctypes.POINTER(RampOptions), P]),
     ("rtkhip_forward_project", I, [P, P, ctypes.POINTER(Image), P, P, ctypes.POINTER(Image), P,
                                    ctypes.POINTER(ctypes.c_longlong), P]),
+    ("rtkhip_forward_project_shape", I, [P, ctypes.POINTER(Image), ctypes.POINTER(Image), PI3]),
     ("rtkhip_back_project", I, [P, P, ctypes.POINTER(Image), P, P, ctypes.POINTER(Image), P, I, I, P]),
     ("rtkhip_joseph_back_project", I, [P, P, ctypes.POINTER(Image), P, P, ctypes.POINTER(Image), P, I, P]),
     ("rtkhip_cg_reconstruct", I, [P, P, ctypes.POINTER(Image), P, ctypes.POINTER(Image), P, P, I, D, I, I, PD,

@@ -148,6 +148,11 @@ private:
   size_t m_Size = 0;
 };
 
+// The column kernel's (columns a workgroup, rows a lane, 64 heights of a run) that the Joseph
+// forward projector takes for these arguments; zeros where it goes ray by ray.  Host only.
+void JosephColumnShape(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vol, const double * source,
+                       const double vol_spacing[3], int shape[3]);
+
 // Makes sure a device is usable before the first launch; maps "no device" to a status.
 void RequireDevice();
 

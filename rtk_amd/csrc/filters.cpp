@@ -928,6 +928,21 @@ rtkhip_forward_project(rtkhip_context * c, const rtkhip_geometry * g, const rtkh
 }
 
 extern "C" int
+rtkhip_forward_project_shape(const rtkhip_geometry * g, const rtkhip_image * stack, const rtkhip_image * vol,
+                             int shape[3])
+{
+  return Guard([&] {
+    RTKHIP_REQUIRE(shape, RTKHIP_ERR_INVALID_ARGUMENT, "forward_project_shape: null argument");
+    CheckImage(vol, "forward_project_shape volume");
+    CheckImage(stack, "forward_project_shape projections");
+    CheckGeometry(g, *stack, true);
+    std::vector<double> p2v, src;
+    JosephRays(*g, *stack, *vol, p2v, src);
+    JosephColumnShape(stack->size, vol->size, p2v.data(), src.data(), vol->spacing, shape);
+  });
+}
+
+extern "C" int
 rtkhip_fft_ramp_filter(rtkhip_context * c, const rtkhip_image * stack, const float * dev_in, float * dev_out,
                        const rtkhip_ramp_options * ramp, void * stream)
 {

@@ -2237,17 +2237,28 @@ CheckArgs(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vo
 }
 
 // Columns a workgroup (W), rows per lane (Q) and profile heights per lane (E) of
-// joseph_fp_column_kernel: the candidates whose 64 E heights hold 64 Q rows at the geometry's largest row step and four
-// heights for the floor and the neighbours above and below.
+// joseph_fp_column_kernel: the candidates whose 64 E heights hold 64 Q rows at the geometry's
+// largest row step and four heights for the floor and the neighbours above and below; q = 0:
+// ray by ray.
 struct ColumnShape
 {
   int w = 0, q = 0, e = 0;
 };
 #define RTKHIP_COLUMN_SHAPES(X)                                                                                      \
   X(4, 1, 1) X(4, 1, 2) X(8, 1, 2) X(8, 2, 2) X(8, 2, 3) X(8, 3, 2) X(8, 3, 3) X(8, 3, 4) X(8, 4, 3) X(8, 4, 4)
-ColumnShape
-ChooseColumnShape(double maxRowStep, int nu, int nv, int np)
+
+// Heights of a column in the y-fastest copy: a zero below and one above the volume, at least
+// one run, whole 16-byte chunks.
+size_t
+ColumnPitch(const ColumnShape & shape, int ny)
 {
+  return std::max<size_t>(64 * size_t(std::max(shape.e, 1)), (size_t(ny) + 5) & ~size_t(3));
+}
+
+ColumnShape
+ChooseColumnShape(double maxRowStep, const int proj_dim[3], const int vol_dim[3])
+{
+  const int nu = proj_dim[0], nv = proj_dim[1], np = proj_dim[2];
   // Larger steps keep the per-ray kernel: fewer than 1.4 rows a voxel share a profile, and
   // that kernel's sums round the positions otherwise, which a 16-bit CG stack (FP(P)
   // rounded to 16 bits) turns into whole steps of its pixels.
@@ -2271,6 +2282,11 @@ ChooseColumnShape(double maxRowStep, int nu, int nv, int np)
 #define RTKHIP_CONSIDER(WW, QQ, EE) consider(WW, QQ, EE);
   RTKHIP_COLUMN_SHAPES(RTKHIP_CONSIDER)
 #undef RTKHIP_CONSIDER
+  // Flat volumes, whose copy would be far larger than they are, keep the per-ray kernel.
+  const size_t nvox = size_t(vol_dim[0]) * vol_dim[1] * vol_dim[2];
+  const size_t padded = ColumnPitch(best, vol_dim[1]) * vol_dim[0] * vol_dim[2];
+  if (padded >= (size_t(1) << 32) || padded > 4 * nvox + (size_t(1) << 24) || vol_dim[2] > 65535)
+    best = ColumnShape{};
   return best;
 }
 
@@ -2303,6 +2319,21 @@ UploadViews(int np, const double * proj_to_vol, const double * source, hipStream
 }
 
 } // namespace
+
+void
+JosephColumnShape(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vol, const double * source,
+                  const double vol_spacing[3], int shape[3])
+{
+  CheckArgs(proj_dim, vol_dim, proj_to_vol, source, vol_spacing);
+  GatherPlan  G;
+  ColumnShape c;
+  if (proj_dim[2] > 0 && PlanGather(proj_dim, vol_dim, proj_to_vol, source, 0., 1., G))
+    c = ChooseColumnShape(G.maxRowStep, proj_dim, vol_dim);
+  shape[0] = c.w;
+  shape[1] = c.q;
+  shape[2] = c.e;
+}
+
 } // namespace rtkhip
 
 extern "C" int
@@ -2359,14 +2390,10 @@ rtkhip_joseph_forward_project(const int proj_dim[3], const int vol_dim[3], const
       ColumnShape shape;
       if (PrepareGather(proj_dim, vol_dim, proj_to_vol, source, inferior_clip, superior_clip, s, freeRows,
                         &maxRowStep) >= 0)
-        shape = ChooseColumnShape(maxRowStep, nu, nv, np);
-      // heights of a column in the y-fastest copy: a zero below and one above the volume, at
-      // least one run, whole 16-byte chunks.  Flat volumes, whose copy would be far larger
-      // than they are, keep the per-ray kernel.
-      const size_t pitch = std::max<size_t>(64 * size_t(std::max(shape.e, 1)), (size_t(vol_dim[1]) + 5) & ~size_t(3));
-      const size_t padded = pitch * vol_dim[0] * vol_dim[2];
-      if (shape.q && padded < (size_t(1) << 32) && padded <= 4 * nvox + (size_t(1) << 24) && vol_dim[2] <= 65535)
+        shape = ChooseColumnShape(maxRowStep, proj_dim, vol_dim);
+      if (shape.q)
       {
+        const size_t pitch = ColumnPitch(shape, vol_dim[1]), padded = pitch * vol_dim[0] * vol_dim[2];
         dT.Resize(padded);
         dim3 tg((vol_dim[0] + 31) / 32, unsigned((pitch + 31) / 32), vol_dim[2]);
         hipLaunchKernelGGL(transpose_xy_kernel, tg, dim3(256), 0, s, dev_vol, dT.get(), vol_dim[0], vol_dim[1],
