@@ -2239,13 +2239,14 @@ CheckArgs(const int proj_dim[3], const int vol_dim[3], const double * proj_to_vo
 // Columns a workgroup (W), rows per lane (Q) and profile heights per lane (E) of
 // joseph_fp_column_kernel: the candidates whose 64 E heights hold 64 Q rows at the geometry's
 // largest row step and four heights for the floor and the neighbours above and below; q = 0:
-// ray by ray.
+// ray by ray.  For Q = 1, 2 and 4 the smallest run that holds 64 Q rows at the largest step
+// taken is the only one compiled: a longer one costs more and is never chosen.
 struct ColumnShape
 {
   int w = 0, q = 0, e = 0;
 };
 #define RTKHIP_COLUMN_SHAPES(X)                                                                                      \
-  X(4, 1, 1) X(4, 1, 2) X(8, 1, 2) X(8, 2, 2) X(8, 2, 3) X(8, 3, 2) X(8, 3, 3) X(8, 3, 4) X(8, 4, 3) X(8, 4, 4)
+  X(4, 1, 1) X(8, 2, 2) X(8, 3, 2) X(8, 3, 3) X(8, 4, 3)
 
 // Heights of a column in the y-fastest copy: a zero below and one above the volume, at least
 // one run, whole 16-byte chunks.
