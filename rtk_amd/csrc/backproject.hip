@@ -269,7 +269,9 @@ UpdateGeneral(const ViewCoef & c, bool itk, const TP * pp, int nu, int nv, float
 // footprint lies inside the detector (one comparison per block) runs with no border test,
 // about 32 instructions an update, others test and clamp every tap; both read the stage.
 // Footprints larger than the stage and optimized views among tilted ones read global memory
-// voxel by voxel.  Same sums as a thread per voxel in global memory, bit for bit.
+// voxel by voxel.  Every update is rounded as by a thread per voxel in global memory; the sums
+// start from zero and the input volume is added last, so with one they may differ from
+// bp_voxel_kernel's in the last bit.
 // VALU-bound; 203 x 181 x 221 <- 157 x 301 x 257, FP16 stack: 3.24 ms (a thread per voxel,
 // every tap from global memory) -> 1.7 ms (750 G updates/s).
 template <typename TP, bool FDK, int NJ, bool VEC, bool TILT>
@@ -305,7 +307,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
 
   // positions along y, and the choice between the tested and the untested column loop (they
   // round differently), are those of blocks of 16 heights for either NJ, so NJ does not show
-  // in the result; jr: this block's first height among the 16
+  // in the result while the view's footprint fits the stage for both (48 rows for 16 heights,
+  // 32 for fewer); jr: this block's first height among the 16
   const int   jr = NJ == 16 ? 0 : j0 & 15;
   const float x = float(i) - ci, z = float(k) - ck, y0 = float(j0) - cj, y16 = float(j0 - jr) - cj;
   const bool  full16 = NJ == 16 ? jn == NJ : j0 - jr + 16 <= ny;
@@ -424,7 +427,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
         auto          coords = [&](int jj, float & rw, float & u, float & v) {
           const float y = y0 + float(jj);
           // the reciprocal's one Newton step is its correctly rounded value (Markstein 1990:
-          // from an approximation within an ulp), what a division gives
+          // from an approximation within an ulp, and unless w's significand is all ones, where
+          // it can be an ulp off), what a division gives
           const float w = fmaf(c.c[11], z, fmaf(c.c[10], y, bw)), r = __builtin_amdgcn_rcpf(w);
           rw = fmaf(fmaf(-w, r, 1.f), r, r);
           u = fmaf(c.c[3], z, fmaf(c.c[2], y, bu)) * rw;
@@ -620,10 +624,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILT ? 5 : 
 }
 
 // The smallest tilted volumes, a thread per voxel: too few for blocks, whose views follow each
-// other behind a barrier each, and a stack that the L2s hold.  Same sums as the blocks'.
+// other behind a barrier each.  The updates are the blocks' (they add the input volume last).
 // Blocks / per voxel, whole calls, ms: FDK 84 x 72 x 76 <- 249 .66 / .40, 92 x 60 x 89 <- 274
 // .65 / .50; CG 91 x 86 x 80 <- 73 .62 / .57; FDK 93 x 82 x 90 <- 294 .73 / .76, 124 x 76 x
-// 109 <- 119 .49 / .54.
+// 109 <- 119 .49 / .54.  The volume decides more than the stack: 64^3 <- 180 x 64^2 .28 / .18,
+// <- 360 x 512^2 1.47 / .91 (FP16 1.63 / .61); 80 x 70 x 90 the same two .26 / .21, 1.46 / 1.13
+// (FP16 1.74 / .81); 86^3 (just below the line) .30 / .27, 1.60 / 1.75 (FP16 1.88 / 1.42), and
+// <- 360 x 256^2, where blocks would do better, .60 / .93.
 constexpr long kPerVoxel = 640L << 10;
 template <typename TP, bool FDK>
 __global__ __launch_bounds__(256) void bp_voxel_kernel(const ViewCoef * __restrict__ views,

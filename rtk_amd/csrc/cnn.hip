@@ -119,6 +119,8 @@ __global__ __launch_bounds__(256) void conv_in_kernel(const float * __restrict__
 // and stores 8 bytes.  256^3 layer: 1.87 ms (497 TFLOP/s; a fragment per tap and output row,
 // LDS-bound) -> 1.08 ms (860 TFLOP/s; the matrix units alone need 0.37, the rest is staging,
 // which one other workgroup per CU overlaps).
+// Rows 8 / 4, a whole inference: 256^3 4.8 ms / 5.6 (where blocks fill the chip; by 128^3 .63 /
+// .71 and 64^3 .112 / .137), 48^3 .081 / .080, 32^3 (64 workgroups of 8) .070 / .057.
 constexpr int kRowsY = 8;
 
 template <bool RELU, bool MASK>
@@ -270,7 +272,7 @@ HasInf(const bf16x8 & v)
 // wavefronts write P of the 18 x 18 halo to LDS, then each thread adds 9 values to each of the
 // three outputs the plane feeds, which it keeps in registers; the next plane's activations are
 // loaded meanwhile.  Every activation is read 1.3 times instead of 27.
-// 256^3: 1.65 ms (864 VALU FMAs and 108 cached 16-byte loads a voxel) -> 0.27 ms.
+// 256^3: 1.65 ms (864 VALU FMAs and 108 cached 16-byte loads a voxel) -> 0.28 ms.
 constexpr int kOutX = 16, kOutHX = kOutX + 2, kOutVox = kOutHX * kOutHX; // halo plane
 constexpr int kOutGroups = (kOutVox + 15) / 16;
 constexpr int kOutStride = 340; // floats of a tap's plane: 4 taps further is 16 LDS banks on

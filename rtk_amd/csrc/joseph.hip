@@ -1467,8 +1467,9 @@ __global__ __launch_bounds__(256) void joseph_gather_shell_kernel(
 // two of its values (a wavefront's LDS accesses complete in order: no barrier).  What a
 // slice needs besides (a, b, fx, offsets: FP64 geometry) is computed for 64 slices at once,
 // one slice per lane, and read back from LDS; the runs of the next kBatch slices are in
-// flight while the current ones are summed.  Heights are FP32 relative to the lowest of each
-// group of 64 rows.  Per slice about 20 + 2 E instructions for the profile and 8 per ray, so
+// flight while the current ones are summed.  Heights are FP32, a + b jv less a whole number
+// per group of 64 rows: a is the height at row 0, so its rounding and b's grow with the row, to
+// 3e-5 voxel at row 960 of 0.52-voxel steps.  Per slice about 20 + 2 E instructions for the profile and 8 per ray, so
 // several rows per lane share one profile.
 // W adjacent columns make a workgroup.  Their runs overlap (X a fraction of a voxel apart),
 // and they are kept within 16 slices of each other by a barrier, so that they share them in
@@ -1792,8 +1793,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(Q <= 2 ?
       // the run of 64 E heights from ylo, one below the band's lowest (a height rounded below
       // the volume reads the zero there), holds every height of the band in the volume
       const int      ylo = min(max(int(floor(fmin(ya, yb))), 0) - 1, pitch - 1 - 64 * E);
-      // each group of 64 rows takes its heights relative to its own lowest, so their FP32
-      // values stay small; rel: that height in the run, 16 bits a group
+      // each group of 64 rows takes its heights less its lowest one's floor, as the coefficients
+      // of the row's number in the whole column (the row's number within the group would round
+      // less, but otherwise than the projections that a 16-bit CG stack was made from: see
+      // ChooseColumnShape); rel: that floor in the run, 16 bits a group
       unsigned rel[2] = { 0, 0 };
       auto *   gl = geom[wave][lane];
 #pragma unroll
@@ -2260,9 +2263,10 @@ ColumnShape
 ChooseColumnShape(double maxRowStep, const int proj_dim[3], const int vol_dim[3])
 {
   const int nu = proj_dim[0], nv = proj_dim[1], np = proj_dim[2];
-  // Larger steps keep the per-ray kernel: fewer than 1.4 rows a voxel share a profile, and
-  // that kernel's sums round the positions otherwise, which a 16-bit CG stack (FP(P)
-  // rounded to 16 bits) turns into whole steps of its pixels.
+  // Larger steps (above 0.714 voxel) keep the per-ray kernel: fewer than 1.4 rows a voxel share
+  // a profile, and that kernel's sums round the positions otherwise, which a 16-bit CG stack
+  // (FP(P) rounded to 16 bits) turns into whole steps of its pixels.  Plain projections and
+  // FP32 stacks do not need that line; runs for larger steps have not been measured.
   ColumnShape best;
   if (maxRowStep * 63. * (1. + 1e-4) + 3. > 48.)
     return best;

@@ -1273,8 +1273,10 @@ rtkhip_ramp_filter(const int proj_dim[3], int xpad, const double * kernel, int t
           im = c ? -kernel[2 * h + 1] : kernel[2 * h + 1];
         },
         s);
-      // pairs of rows per workgroup: a butterfly of the largest radix for most threads, in
-      // at most 40 KB of LDS (four workgroups per CU); the twiddles beside them where they fit
+      // pairs of rows per workgroup: a butterfly of the largest radix for most threads, where
+      // more than one pair fits 40 KB of LDS; the twiddles beside them where the sum is at most
+      // 64 KB.  N = 605: four pairs, 43 KB, three workgroups per CU; 2002: one, 47 KB, three; 2500:
+      // one, 59 KB, two
       const int    maxRadix = *std::max_element(radices.begin(), radices.end());
       const int    F = int(std::max<size_t>(
         1, std::min<size_t>((256 * maxRadix + N / 2) / N, (size_t(40) << 10) / (sizeof(float2) * 2 * size_t(N)))));
