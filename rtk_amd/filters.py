@@ -139,13 +139,15 @@ class Image:
     def descriptor(self):
         # whole arrays at a time: 1.4 us, 3.8 element by element (a call has two or three)
         d = _lib.Image()
-        d.size[:], d.index[:] = self.size, self.index[:3]
-        d.origin[:], d.spacing[:] = self.origin[:3], self.spacing[:3]
+        d.size[:], d.index[:] = self.size, tuple(self.index[:3])
+        d.origin[:], d.spacing[:] = tuple(self.origin[:3]), tuple(self.spacing[:3])
         return d
 
     def like(self, tensor):
         if tensor.dim() != 3:
             raise ValueError("Image expects a 3-D tensor [z, y, x]")
+        if not (type(self.origin) is type(self.spacing) is type(self.index) is tuple):
+            return Image(tensor, self.origin, self.spacing, self.index)  # set since to something else
         image = Image.__new__(Image)  # the meta-data is in its final form already
         image.tensor = tensor.contiguous()
         image.origin, image.spacing, image.index = self.origin, self.spacing, self.index
