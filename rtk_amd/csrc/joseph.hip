@@ -325,7 +325,7 @@ struct Walker
   {
     int cix, ciy;
     Stage2D(R, cix, ciy, lx, ly);
-    return cix + ciy * R.oy; // 32 bits: a z row of a y-dominant ray may be 2^24 voxels and more
+    return cix + ciy * R.oy; // 32 bits: y-dominant rays step by z planes, up to 2^30 voxels
   }
   // Lower-left tap (cix, ciy) of the current sample, then advance one slice.
   __device__ __forceinline__ void Stage2D(const Ray & R, int & cix, int & ciy, float & lx, float & ly)
